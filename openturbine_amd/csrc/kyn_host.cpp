@@ -838,6 +838,16 @@ double* field_ptr(kyn_system_s* s, int field, int& width) {
     }
 }
 
+// Whether a fused launch of num_models models gives every block a workgroup of its own: while the
+// models are no more than the workgroups the chip holds (one per CU in FP64, two in FP32).  Beyond
+// that the models fill it by themselves, and a block that waits for a larger one of its model holds
+// a place another model could use.  Measured, 3-blade rotors of mixed blade sizes, us per step
+// unsplit / split: FP64 96 rotors 2940 / 1442, 256 2963 / 2725, 300 3132 / 3275, 512 4247 / 5239;
+// FP32 96 2303 / 942, 256 2330 / 1498, 512 2442 / 2328, 700 2914 / 3142, 1536 5028 / 6526.
+bool fused_split_models(size_t num_models, int cus, bool fp32) {
+    return num_models <= static_cast<size_t>(cus) * (fp32 ? 2 : 1);
+}
+
 int zoff_host(const kyn_system_s* s, int b) {
     int off = 0;
     for (size_t k = 0; k < s->large_blocks.size(); ++k) {
@@ -964,6 +974,9 @@ void check_device_errors(kyn_system_s* s) {
     if (flags == 0) return;
     const int zero = 0;
     hip_check(hipMemcpy(s->S.dev_error, &zero, sizeof(int), hipMemcpyHostToDevice), "H2D");
+    if (!(flags & kyn::kDevErrLuWait))
+        throw KynError(KYN_ERR_HIP, "a workgroup of the fused step gave up waiting for the other blocks of its model; "
+                                    "the step's results are invalid");
     throw KynError(KYN_ERR_HIP, "a wave of the blocked LU gave up waiting on its look-ahead counter "
                                 "(bound " + std::to_string(s->S.lu_wait_limit) + " polls); the step's results are invalid");
 }
@@ -1250,16 +1263,37 @@ kyn_system kyn_system_create(const kyn_model* models, size_t num_models, const k
         S.model_gravity = Ar.up(B.model_gravity);
         S.model_load_begin = Ar.zeros<int>(num_models + 1);
         {
-            // dispatch order of the fused launch: longest expected step first (sum over the model's
-            // blocks of n^2, between the panel's O(n) and the trailing update's O(n^3)), so the
-            // short models fill the tail of the grid
+            // the fused launch's list: longest expected step first (sum over the model's blocks of
+            // n^2, between the panel's O(n) and the trailing update's O(n^3)), so the short models
+            // fill the tail of the grid
             std::vector<double> cost(num_models, 0.);
             for (size_t b = 0; b < B.block_n.size(); ++b)
                 cost[B.block_model[b]] += static_cast<double>(B.block_n[b]) * B.block_n[b];
             std::vector<int> order(num_models);
             for (size_t m = 0; m < num_models; ++m) order[m] = static_cast<int>(m);
             std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return cost[x] > cost[y]; });
-            S.model_order = Ar.up(order);
+            // One workgroup per block where the models do not fill the chip by themselves (see
+            // fused_split_models for the line); every block of a split model must be able to run at once
+            int cus = 0;
+            hip_check(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev), "attr");
+            const bool split_all = sys->exec_mode == KYN_EXEC_FUSED && fused_split_models(num_models, cus, S.precision != 0);
+            std::vector<int> work;
+            bool split = false;
+            for (int m : order) {
+                const int nb = B.model_block_end[m] - B.model_block_begin[m];
+                if (split_all && nb > 1 && nb <= std::min(kyn::kMaxSplitBlocks, cus)) {
+                    split = true;
+                    for (int k = 0; k < nb; ++k) work.insert(work.end(), {m, k});
+                } else {
+                    work.insert(work.end(), {m, -1});
+                }
+            }
+            S.fused_work = Ar.up(work);
+            S.num_fused_work = static_cast<int>(work.size() / 2);
+            S.fused_ticket = split ? Ar.zeros<int>(1) : nullptr;
+            S.fused_xch = split ? Ar.up(std::vector<unsigned long long>(B.block_n.size() * static_cast<size_t>(S.p.max_iter),
+                                                                       kyn::kXchEmpty))
+                                : nullptr;
         }
         S.block_model = Ar.up(B.block_model);
         S.block_n = Ar.up(B.block_n);

@@ -1773,26 +1773,40 @@ __device__ __forceinline__ void times_tangent(const double* g, const double* trr
 // ---------------------------------------------------------------------------------------
 // Schedule application (device-resident per-step inputs)
 // ---------------------------------------------------------------------------------------
-__device__ __forceinline__ void apply_schedule_model(const DevSys& S, int m) {
+// mine(node): whether this workgroup applies the inputs of a node (and of the constraints on it)
+template <typename Mine>
+__device__ __forceinline__ void apply_schedule_model(const DevSys& S, int m, Mine mine) {
     if (S.sched_steps <= 0) return;
     const int slot = *S.sched_slot;
     if (slot >= S.sched_steps) return;
     if (S.sched_cdisp)
         for (int c = S.model_con_begin[m] + (int)threadIdx.x; c < S.model_con_end[m]; c += blockDim.x)
+            if (mine(S.con_target[c]))
 #pragma unroll
-            for (int k = 0; k < 7; ++k)
-                S.con_input[c * 7 + k] = S.sched_cdisp[((size_t)slot * S.num_cons + c) * 7 + k];
+                for (int k = 0; k < 7; ++k)
+                    S.con_input[c * 7 + k] = S.sched_cdisp[((size_t)slot * S.num_cons + c) * 7 + k];
     if (S.sched_loads)
         for (int k = S.model_load_begin[m] + (int)threadIdx.x; k < S.model_load_begin[m + 1]; k += blockDim.x) {
             const int node = S.sched_load_nodes[k];
+            if (!mine(node)) continue;
 #pragma unroll
             for (int c = 0; c < 6; ++c)
                 S.f[node * 6 + c] = S.sched_loads[((size_t)slot * S.sched_num_loaded + k) * 6 + c];
         }
 }
 
+// After a step: the schedule's next row, and the split launch's ticket and exchange slots cleared
+// for the next step (thread per block; the slots its model's iterations used, all of them after a
+// wait that gave up).
 __global__ void k_advance_slot(DevSys S) {
-    if (threadIdx.x == 0 && blockIdx.x == 0 && S.sched_steps > 0) *S.sched_slot += 1;
+    const int g = blockIdx.x * blockDim.x + threadIdx.x;
+    if (g == 0 && S.sched_steps > 0) *S.sched_slot += 1;
+    if (S.fused_ticket == nullptr) return;
+    if (g == 0) *S.fused_ticket = 0;
+    if (g < S.num_blocks) {
+        const int used = *S.dev_error != 0 ? S.p.max_iter : S.model_iters[S.block_model[g]];
+        for (int k = 0; k < used; ++k) S.fused_xch[(size_t)g * S.p.max_iter + k] = kXchEmpty;
+    }
 }
 
 // ---------------------------------------------------------------------------------------
@@ -2181,13 +2195,81 @@ __device__ __forceinline__ void factor_solve_uncondition(const DevSys& S, int b,
 }
 
 // ---------------------------------------------------------------------------------------
-// Fused form: one workgroup per model, one launch per time step
+// Fused form: one launch per time step, one workgroup per model, or one per block of a model
+// where the models alone leave the chip idle (the launch list fused_work, built at setup).
+//
+// Split models: a model's blocks share nothing but the convergence error, so each block's Newton
+// loop runs in a workgroup of its own, and per iteration the workgroups exchange one number: each
+// stores its block's error sum into the slot (block, iteration) and reads the others', summed
+// in block order, so every workgroup takes the same decision and all results are those of the
+// unsplit form bit for bit.  The number is the only thing one reads of another, so the exchange is
+// a relaxed device-scope store and load of one 64-bit word (an empty slot holds kXchEmpty).
+// Workgroups take their list entry by ticket in the order they start and a model's entries are
+// consecutive: whoever waits, the earliest unfinished model's workgroups are all running or the
+// next to start, so every wait ends (the host splits only models with no more blocks than the
+// chip has CUs).  The wait is bounded all the same.
+// Measured, us per step unsplit / split: one 3-blade rotor, FP64 2597 / 1061, FP32 1989 / 834; 96
+// rotors of mixed blade sizes, FP64 2940 / 1442, FP32 2303 / 942.
 // ---------------------------------------------------------------------------------------
+// Whether the workgroup of a split model's block owns a node: its block's, and the first
+// block's workgroup also the nodes of no block.
+__device__ __forceinline__ bool owns_node(const DevSys& S, int node, int part, int block) {
+    const int nb = S.node_block[node];
+    return nb < 0 ? part == 0 : nb == block;
+}
+
+// Publishes this block's error sum of one iteration and returns the model's, through red[0]; false
+// when the wait for the other blocks gave up.
+__device__ __forceinline__ bool exchange_err_sum(const DevSys& S, int b0, int nb, int b, int iter, double own, double* red,
+                                                 double& sum) {
+    const int t = threadIdx.x;
+    if (t < 64) {
+        unsigned long long* slot = S.fused_xch + iter;
+        if (t == 0) {
+            unsigned long long w = (unsigned long long)__double_as_longlong(own);
+            if (w == kXchEmpty) w = 0x7ff8000000000000ull;  // any NaN does
+            __hip_atomic_store(slot + (size_t)b * S.p.max_iter, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        unsigned long long w = t < nb ? kXchEmpty : 0;
+        int polls = 0;
+        for (;; ++polls) {
+            if (w == kXchEmpty)
+                w = __hip_atomic_load(slot + (size_t)(b0 + t) * S.p.max_iter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (!__any(w == kXchEmpty)) break;
+            if (polls >= kPeerWaitLimit) {
+                if (t == 0) __hip_atomic_fetch_or(S.dev_error, kDevErrPeerWait, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                break;
+            }
+            __builtin_amdgcn_s_sleep(4);
+        }
+        const double v = __longlong_as_double((long long)w);
+        double acc = 0.;
+        for (int k = 0; k < nb; ++k) acc += rdlane(v, k);
+        if (t == 0) {
+            red[0] = acc;
+            red[1] = polls < kPeerWaitLimit ? 1. : 0.;
+        }
+    }
+    __syncthreads();
+    sum = red[0];
+    return red[1] != 0.;
+}
+
+// The kernel's first argument, read anew from the kernel-argument segment: what is loaded through
+// the reference stays below this point.  (Through the argument itself the compiler loads every
+// pointer of the struct once, before the Newton loop, and keeps ~800 scalar registers spilled.)
+__device__ __forceinline__ const DevSys& sys_args() {
+    typedef const __attribute__((address_space(4))) DevSys* arg_ptr;
+    arg_ptr p = (arg_ptr)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(const DevSys*)p;
+}
+
 template <typename TT>
-__device__ __forceinline__ void fused_step_body(const DevSys& S, int Nm, int Qm, int nm) {
+__device__ __forceinline__ void fused_step_body(int Nm, int Qm, int nm) {
     extern __shared__ __align__(16) char sm[];
+    const DevSys& S = sys_args();
     const Lay L = make_layout(Nm, Qm, nm, S.max_block_cons, S.refine_sweeps > 0, (int)sizeof(TT), true);
-    const int m = S.model_order[blockIdx.x];
     const int t = threadIdx.x;
     double* red = reinterpret_cast<double*>(sm + L.red);
     int* misc = reinterpret_cast<int*>(sm + L.misc);
@@ -2196,55 +2278,80 @@ __device__ __forceinline__ void fused_step_body(const DevSys& S, int Nm, int Qm,
     double* xs2 = reinterpret_cast<double*>(sm + L.xs2);
     int* piv = reinterpret_cast<int*>(sm + L.piv);
     TT* A = reinterpret_cast<TT*>(sm + L.A);
-    const StepConsts& p = S.p;
+
+    int g = blockIdx.x;
+    if (S.fused_ticket != nullptr) {  // uniform
+        if (t == 0) misc[0] = atomicAdd(S.fused_ticket, 1);
+        __syncthreads();
+        g = __builtin_amdgcn_readfirstlane(misc[0]);
+    }
+    const int m = S.fused_work[2 * g], part = S.fused_work[2 * g + 1];  // part: block within the model, -1: all
+    const int mb0 = S.model_block_begin[m], mb1 = S.model_block_end[m];
+    const int b0 = part < 0 ? mb0 : mb0 + part, b1 = part < 0 ? mb1 : b0 + 1;
+    const bool lead = part <= 0;  // writes the model's bookkeeping
+    auto mine = [&](int node) { return part < 0 || owns_node(S, node, part, b0); };
 
     // inputs, PredictNextState, ResetConstraints (step.hpp:49-50)
-    apply_schedule_model(S, m);
+    apply_schedule_model(S, m, mine);
     __syncthreads();
     for (int node = S.model_node_begin[m] + t; node < S.model_node_end[m]; node += blockDim.x)
-        predict_node(S, node);
+        if (mine(node)) predict_node(S, node);
     for (int c = S.model_con_begin[m] + t; c < S.model_con_end[m]; c += blockDim.x)
+        if (mine(S.con_target[c]))
 #pragma unroll
-        for (int k = 0; k < 6; ++k) {
-            S.con_lambda[c * 6 + k] = 0.;
-            S.con_sys_res[c * 6 + k] = 0.;
-        }
+            for (int k = 0; k < 6; ++k) {
+                S.con_lambda[c * 6 + k] = 0.;
+                S.con_sys_res[c * 6 + k] = 0.;
+            }
     __syncthreads();
 
     const double ndofs = (double)S.model_ndofs[m];
+    const int max_iter = S.p.max_iter;
     int converged = 0;
     int iter = 0;
     double err_prev = __builtin_inf();  // convergence error of the previous Newton iteration
-    for (; iter < p.max_iter; ++iter) {
-        // FP64 refinement of the FP32 solve where it decides the final state: the Newton
-        // increments contract by ~20x per iteration, so a solve error matters only in the last
-        // iterations, whose predecessors' errors are small (an inexact-Newton forcing rule)
-        const bool refine_now = S.refine_sweeps > 0 && (S.refine_err_bound <= 0. || err_prev < S.refine_err_bound);
+    for (; iter < max_iter; ++iter) {
         double err_sum = 0.;
-        for (int b = S.model_block_begin[m]; b < S.model_block_end[m]; ++b) {
-            const int n = S.block_n[b];
-            const int e = S.block_elems[S.block_elem_begin[b]];
+        for (int b = b0; b < b1; ++b) {
             KYN_PHASE_MARK(0);
-            // every system row starts at -f (a node outside the element, e.g. a massless hub,
-            // takes only its load and constraint terms); the element rows are then written as
-            // -f + R after the element phase's first barrier
-            for (int i = t; i < S.block_nsys[b]; i += blockDim.x)
-                rhs[i] = -S.f[S.block_nodes[S.block_node_begin[b] + i / 6] * 6 + i % 6];
-            element_phase<TT, true>(S, e, sm, L, n, nullptr, nullptr, m);
+            int n;
+            {
+                const DevSys& S = sys_args();
+                n = S.block_n[b];
+                const int e = S.block_elems[S.block_elem_begin[b]];
+                // every system row starts at -f (a node outside the element, e.g. a massless hub,
+                // takes only its load and constraint terms); the element rows are then written as
+                // -f + R after the element phase's first barrier
+                for (int i = t; i < S.block_nsys[b]; i += blockDim.x)
+                    rhs[i] = -S.f[S.block_nodes[S.block_node_begin[b] + i / 6] * 6 + i % 6];
+                element_phase<TT, true>(S, e, sm, L, n, nullptr, nullptr, m);
+            }
             KYN_PHASE_MARK(5);
-            block_constraints<TT>(S, b, sm, L);
-            condition_rhs(S, b, rhs);
+            block_constraints<TT>(sys_args(), b, sm, L);
+            condition_rhs(sys_args(), b, rhs);
             KYN_PHASE_MARK(6);
-            // unfactored copy for refinement: row-major, row stride (n + 3) & ~3, at the block's own offset
-            TT* Ac = (S.Acopy != nullptr && refine_now) ? reinterpret_cast<TT*>(S.Acopy) + S.block_C_off[b] : nullptr;
-            factor_solve_uncondition<TT>(S, b, A, Ac, L.lda, piv, rhs, xs, xs2, sm, L);
+            {
+                const DevSys& S = sys_args();
+                // FP64 refinement of the FP32 solve where it decides the final state: the Newton
+                // increments contract by ~20x per iteration, so a solve error matters only in the
+                // last iterations, whose predecessors' errors are small (an inexact-Newton forcing
+                // rule)
+                const bool refine_now =
+                    S.refine_sweeps > 0 && (S.refine_err_bound <= 0. || err_prev < S.refine_err_bound);
+                // unfactored copy for refinement: row-major, row stride (n + 3) & ~3, at the block's own offset
+                TT* Ac =
+                    (S.Acopy != nullptr && refine_now) ? reinterpret_cast<TT*>(S.Acopy) + S.block_C_off[b] : nullptr;
+                factor_solve_uncondition<TT>(S, b, A, Ac, L.lda, piv, rhs, xs, xs2, sm, L);
+            }
             KYN_PHASE_MARK(10);
-            err_sum += block_error_and_update(S, b, xs, red);
+            err_sum += block_error_and_update(sys_args(), b, xs, red);
             KYN_PHASE_MARK(11);
         }
+        const DevSys& S = sys_args();
+        if (part >= 0 && !exchange_err_sum(S, mb0, mb1 - mb0, b0, iter, err_sum, red, err_sum)) break;
         const double err = sqrt(err_sum / ndofs);
         err_prev = err;
-        if (t == 0) S.err_hist[(size_t)m * p.max_iter + iter] = err;
+        if (t == 0 && lead) S.err_hist[(size_t)m * max_iter + iter] = err;
         // the reference's loop test `err > 1.` (step.hpp:54): a NaN error also ends the loop,
         // and the step then counts as converged
         if (!(err > 1.)) {
@@ -2253,28 +2360,33 @@ __device__ __forceinline__ void fused_step_body(const DevSys& S, int Nm, int Qm,
             break;
         }
     }
-    if (converged) {
-        for (int node = S.model_node_begin[m] + t; node < S.model_node_end[m]; node += blockDim.x)
-            epilogue_node(S, node);
-        for (int c = S.model_con_begin[m] + t; c < S.model_con_end[m]; c += blockDim.x) constraint_output(S, c);
-    }
-    if (t == 0) {
-        S.model_status[m] = converged ? 0 : 1;
-        S.model_iters[m] = iter;
-        S.model_active[m] = 0;
-        S.model_iter_total[m] += iter;
-        S.model_fail_total[m] += converged ? 0 : 1;
+    {
+        const DevSys& S = sys_args();
+        auto mine = [&](int node) { return part < 0 || owns_node(S, node, part, b0); };
+        if (converged) {
+            for (int node = S.model_node_begin[m] + t; node < S.model_node_end[m]; node += blockDim.x)
+                if (mine(node)) epilogue_node(S, node);
+            for (int c = S.model_con_begin[m] + t; c < S.model_con_end[m]; c += blockDim.x)
+                if (mine(S.con_target[c])) constraint_output(S, c);
+        }
+        if (t == 0 && lead) {
+            S.model_status[m] = converged ? 0 : 1;
+            S.model_iters[m] = iter;
+            S.model_active[m] = 0;
+            S.model_iter_total[m] += iter;
+            S.model_fail_total[m] += converged ? 0 : 1;
+        }
     }
 }
 
 // FP64 tangent: the KKT block alone is up to 141 KB of LDS, one workgroup per CU.
 __global__ void __launch_bounds__(kThreads) k_fused_step_f64(DevSys S, int Nm, int Qm, int nm) {
-    fused_step_body<double>(S, Nm, Qm, nm);
+    fused_step_body<double>(Nm, Qm, nm);
 }
 // FP32 tangent: blocks up to 143 dofs fit in 80 KB, so two workgroups share a CU (registers
 // capped at 256 per lane for that).
 __global__ void __launch_bounds__(kThreads, 2) k_fused_step_f32(DevSys S, int Nm, int Qm, int nm) {
-    fused_step_body<float>(S, Nm, Qm, nm);
+    fused_step_body<float>(Nm, Qm, nm);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -2282,7 +2394,7 @@ __global__ void __launch_bounds__(kThreads, 2) k_fused_step_f32(DevSys S, int Nm
 // ---------------------------------------------------------------------------------------
 __global__ void __launch_bounds__(kThreads) k_plain_predict(DevSys S) {
     const int m = blockIdx.x, t = threadIdx.x;
-    apply_schedule_model(S, m);
+    apply_schedule_model(S, m, [](int) { return true; });
     __syncthreads();
     for (int node = S.model_node_begin[m] + t; node < S.model_node_end[m]; node += blockDim.x)
         predict_node(S, node);
@@ -3245,9 +3357,9 @@ hipError_t set_lds_limits(size_t bytes) {
 void launch_fused_step(const DevSys& S, int Nm, int Qm, int nm, hipStream_t st) {
     const size_t lds = fused_lds_bytes(Nm, Qm, nm, S.max_block_cons, S.refine_sweeps, S.precision);
     if (S.precision)
-        hipLaunchKernelGGL(k_fused_step_f32, dim3(S.num_models), dim3(kThreads), lds, st, S, Nm, Qm, nm);
+        hipLaunchKernelGGL(k_fused_step_f32, dim3(S.num_fused_work), dim3(kThreads), lds, st, S, Nm, Qm, nm);
     else
-        hipLaunchKernelGGL(k_fused_step_f64, dim3(S.num_models), dim3(kThreads), lds, st, S, Nm, Qm, nm);
+        hipLaunchKernelGGL(k_fused_step_f64, dim3(S.num_fused_work), dim3(kThreads), lds, st, S, Nm, Qm, nm);
 }
 // ---------------------------------------------------------------------------------------
 // Element-terms scratch of the no-allocation entry point: one element's residual [N][6] and
@@ -3284,7 +3396,8 @@ void launch_element_terms(const DevSys& S, int Nm, int Qm, int e, double* res, d
 }
 
 void launch_advance_slot(const DevSys& S, hipStream_t st) {
-    hipLaunchKernelGGL(k_advance_slot, dim3(1), dim3(64), 0, st, S);
+    const bool split = S.fused_ticket != nullptr;
+    hipLaunchKernelGGL(k_advance_slot, dim3(split ? (S.num_blocks + 63) / 64 : 1), dim3(64), 0, st, S);
 }
 void launch_plain_predict(const DevSys& S, hipStream_t st) {
     hipLaunchKernelGGL(k_plain_predict, dim3(S.num_models), dim3(kThreads), 0, st, S);

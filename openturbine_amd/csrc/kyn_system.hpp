@@ -71,7 +71,12 @@ struct DevSys {
     const int* model_ndofs;
     const double* model_gravity;  // [m][3]
     const int* model_load_begin;  // into sched_load_nodes (sorted by node), [m+1]
-    const int* model_order;       // fused launch: workgroup g runs model model_order[g] (costliest first)
+    // ---- fused launch: workgroup g runs fused_work[2 g] = model (costliest first), fused_work[2 g + 1]
+    //      = the one block of it to run, counted from the model's first, or -1 for all of them
+    const int* fused_work;
+    int num_fused_work;
+    int* fused_ticket;              // split launch (else null): list entries taken by started workgroups
+    unsigned long long* fused_xch;  // split launch: [block][max_iter] error sums, kXchEmpty until stored
 
     // ---- blocks
     const int* block_model;
@@ -237,5 +242,12 @@ struct DevSys {
 
 constexpr int kLuWaitLimitDefault = 1 << 20;  // polls of ~64 cycles: ~28 ms at 2.4 GHz
 constexpr int kDevErrLuWait = 1;
+// split fused launch: an exchange slot nobody has stored to (a NaN that no error sum is stored
+// as), and the polls (~0.2 us each) a workgroup waits for its model's other blocks: seconds, since
+// they may not have started behind another stream's kernels
+constexpr unsigned long long kXchEmpty = ~0ull;
+constexpr int kPeerWaitLimit = 1 << 26;
+constexpr int kDevErrPeerWait = 2;
+constexpr int kMaxSplitBlocks = 64;  // blocks of a split model: one lane each polls a block's slot
 
 }  // namespace kyn
