@@ -19,8 +19,10 @@
 // forming the one R entry of its B operand (contract_mfma_f32).
 #include <hip/hip_runtime.h>
 
+#include <climits>
 #include <cstdint>
 #include <mutex>
+#include <type_traits>
 
 #include "kyn_device.hpp"
 #include "kyn_system.hpp"
@@ -675,13 +677,13 @@ __device__ __forceinline__ void element_phase(const DevSys& S, int e, char* sm, 
 //
 // Right-looking, panels of 16 columns.  Wave 0 factors a panel in registers (lane l holds the
 // rows not yet pivoted, logical c0 + l, c0 + l + 64, ...): per column a candidate per lane, a
-// 64-lane argmax by DPP row exchanges and row broadcasts (FP64: max, then the lowest logical row
-// holding it; FP32: one reduction of a packed magnitude / row key), the pivot row broadcast by
-// readlane, then the in-panel rank-1 update; no barrier inside a panel.  The other waves form
-// the panel's U rows over the trailing columns (forward substitution with the panel's unit L)
-// and update the trailing rows, the next panel's columns first (look-ahead).  Every entry sees
-// the same FMA sequence as in the oracle's unblocked loop (a_ij -= l_ik u_kj for k ascending),
-// so FP64 factors are bit-identical to the oracle's.
+// 64-lane argmax by integer max over DPP row exchanges and row broadcasts (FP64: of the magnitudes'
+// high words, then, where rows share it, low words and rows; FP32: one reduction of a packed
+// magnitude / row key), the pivot row broadcast by readlane, then the in-panel rank-1 update; no
+// barrier inside a panel.  The other waves form the panel's U rows over the trailing columns
+// (forward substitution with the panel's unit L) and update the trailing rows on the matrix cores,
+// the next panel's columns first (look-ahead).  Every entry sees the same sequence of FMAs as in
+// the oracle's unblocked loop (a_ij -= l_ik u_kj for k ascending); see MfmaTile.
 //
 // Pivoting is implicit: rows never move; phys_of maps logical -> physical rows (the position
 // the oracle's dense LU holds a row at after its swaps).  Pivot: largest |a_ik| over
@@ -710,83 +712,22 @@ __device__ __forceinline__ TT* panel_l11(const LuScratch& W, int c0) {
 
 constexpr int kDppRowMirror = 0x140, kDppRowHalfMirror = 0x141, kDppQuad3210 = 0x1B, kDppQuad1032 = 0xB1;
 
-template <int C>
-__device__ __forceinline__ int dpp_x(int v) {
-    return __builtin_amdgcn_update_dpp(0, v, C, 0xF, 0xF, false);
-}
-template <int C>
-__device__ __forceinline__ int lane_x(int v) {
-    return dpp_x<C>(v);
-}
-template <int C>
-__device__ __forceinline__ float lane_x(float v) {
-    return __int_as_float(lane_x<C>(__float_as_int(v)));
-}
-template <int C>
-__device__ __forceinline__ double lane_x(double v) {
-    const long long b = __double_as_longlong(v);
-    const int lo = lane_x<C>((int)(b & 0xffffffffll)), hi = lane_x<C>((int)(b >> 32));
-    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
 // Row broadcasts (GFX9 DPP): lane 15 of each row to the next row (written rows 1 and 3), and
-// lane 31 to rows 2 and 3; rows outside the mask keep `old`.
+// lane 31 to rows 2 and 3; rows outside the mask keep the first operand.
 constexpr int kDppRowBcast15 = 0x142, kDppRowBcast31 = 0x143;
-template <int C, int RM>
-__device__ __forceinline__ int dpp_old(int old, int v) {
-    return __builtin_amdgcn_update_dpp(old, v, C, RM, 0xF, false);
-}
-template <int C, int RM>
-__device__ __forceinline__ float dpp_old(float old, float v) {
-    return __int_as_float(dpp_old<C, RM>(__float_as_int(old), __float_as_int(v)));
-}
-template <int C, int RM>
-__device__ __forceinline__ double dpp_old(double old, double v) {
-    const long long o = __double_as_longlong(old), b = __double_as_longlong(v);
-    const int lo = dpp_old<C, RM>((int)(o & 0xffffffffll), (int)(b & 0xffffffffll));
-    const int hi = dpp_old<C, RM>((int)(o >> 32), (int)(b >> 32));
-    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
-// Reduction over the 64 lanes whose result is valid in lane 63: four in-row exchanges, then the
-// two row broadcasts (no cross-row swaps).
-template <typename T, typename Op>
-__device__ __forceinline__ T wave_reduce_to63(T v, Op op) {
-    v = op(v, lane_x<kDppQuad1032>(v));
-    v = op(v, lane_x<kDppQuad3210>(v));
-    v = op(v, lane_x<kDppRowHalfMirror>(v));
-    v = op(v, lane_x<kDppRowMirror>(v));
-    v = op(v, dpp_old<kDppRowBcast15, 0xA>(v, v));
-    return op(v, dpp_old<kDppRowBcast31, 0xC>(v, v));
-}
 __device__ __forceinline__ int imax(int a, int b) { return a > b ? a : b; }
-__device__ __forceinline__ int imin(int a, int b) { return a < b ? a : b; }
-// max over lanes (to every lane through lane 63)
+// max over lanes (to every lane through lane 63); each step one v_max_i32 with the exchange as
+// its DPP operand (no lane is read from outside its row, and the row broadcasts' masked rows take
+// the identity)
 __device__ __forceinline__ int wave_max(int v) {
-    return __builtin_amdgcn_readlane(wave_reduce_to63(v, imax), 63);
+    v = imax(v, __builtin_amdgcn_update_dpp(0, v, kDppQuad1032, 0xF, 0xF, true));
+    v = imax(v, __builtin_amdgcn_update_dpp(0, v, kDppQuad3210, 0xF, 0xF, true));
+    v = imax(v, __builtin_amdgcn_update_dpp(0, v, kDppRowHalfMirror, 0xF, 0xF, true));
+    v = imax(v, __builtin_amdgcn_update_dpp(0, v, kDppRowMirror, 0xF, 0xF, true));
+    v = imax(v, __builtin_amdgcn_update_dpp(INT_MIN, v, kDppRowBcast15, 0xA, 0xF, false));
+    v = imax(v, __builtin_amdgcn_update_dpp(INT_MIN, v, kDppRowBcast31, 0xC, 0xF, false));
+    return __builtin_amdgcn_readlane(v, 63);
 }
-__device__ __forceinline__ double wave_max(double v) {
-    const double r = wave_reduce_to63(v, [](double a, double b) { return fmax(a, b); });
-    const long long b = __double_as_longlong(r);
-    const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffll), 63), hi = __builtin_amdgcn_readlane((int)(b >> 32), 63);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
-__device__ __forceinline__ int wave_min(int v) {
-    return __builtin_amdgcn_readlane(wave_reduce_to63(v, imin), 63);
-}
-// pivot candidate magnitude: FP32 as the bit pattern of |v| (an int ordered like |v| for
-// non-negative floats, so the reduction is an integer max), FP64 as |v|; -1 = not a candidate
-__device__ __forceinline__ int cand_of(float v, bool ok) { return ok && v == v ? __float_as_int(fabsf(v)) : -1; }
-__device__ __forceinline__ double cand_of(double v, bool ok) { return ok ? fabs(v) : -1.; }
-template <typename TT>
-struct Cand;
-template <>
-struct Cand<float> {
-    using type = int;
-};
-template <>
-struct Cand<double> {
-    using type = double;
-};
-
 __device__ __forceinline__ float rdlane(float v, int l) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
 }
@@ -804,104 +745,133 @@ __device__ __forceinline__ TT slot_tag(TT v) {
     return v;
 }
 
+// bits of b where m is 0, of a where m is -1
+__device__ __forceinline__ float mask_sel(int m, float a, float b) {
+    return __int_as_float((__float_as_int(a) & m) | (__float_as_int(b) & ~m));
+}
+__device__ __forceinline__ double mask_sel(int m, double a, double b) {
+    const unsigned long long x = __double_as_longlong(a), y = __double_as_longlong(b);
+    const unsigned lo = ((unsigned)x & m) | ((unsigned)y & ~m);
+    const unsigned hi = ((unsigned)(x >> 32) & m) | ((unsigned)(y >> 32) & ~m);
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+__device__ __forceinline__ bool is_zero(float v) { return (__float_as_int(v) << 1) == 0; }
+__device__ __forceinline__ bool is_zero(double v) { return (__double_as_longlong(v) << 1) == 0; }
+
 // One pivot column (J) of the wave-0 panel factorization: pivot search over the 64 lanes, pivot
-// row broadcast, multipliers and the rank-1 update of the panel's later columns.
+// row broadcast, multipliers and the rank-1 update of the panel's later columns.  done[s]: -1 for
+// a row that is no candidate (pivoted, or past the block), else 0.
+// A single wave issues about one instruction per four cycles, so a column costs its instruction
+// count: the search is one integer reduction over the magnitudes' high words, masks are bitwise
+// selects on done, and the logical rows are touched only by an interchange.  Panels per block of
+// the mixed FP64 ensemble (n = 42 .. 132): 61k cycles, 79k with reductions of doubles and of row
+// keys; the whole LU 139k -> 105k.
 template <typename TT, int NS, bool kFull, int J>
-__device__ __forceinline__ void panel_columns(TT (&P)[NS][kPanel], int (&lg)[NS], int (&pl)[kPanel], int c0, int w,
-                                              int lane) {
+__device__ __forceinline__ void panel_columns(TT (&P)[NS][kPanel], int (&lg)[NS], int (&done)[NS], int (&pl)[kPanel],
+                                              int c0, int w, int lane) {
     if constexpr (J < kPanel) {
         if (kFull || J < w) {
             const int k = c0 + J;
-            int key;
+            unsigned long long bm[NS];  // ballots with the pivot row's lane in its slot
             if constexpr (sizeof(TT) == 4) {
                 // FP32: one reduction of (|a_rk| to 15 mantissa bits, 255 - logical row): the
                 // largest magnitude, and among magnitudes equal to 2^-15 the lowest logical row
-                // (NaN never wins; no candidate or a NaN a_kk keeps row k); the physical row of
-                // the winner from a ballot
+                // (NaN never wins; no candidate or a NaN a_kk keeps row k); the winner's lane
+                // from a ballot
                 int bk = -1;
                 bool dnan = false;
 #pragma unroll
                 for (int s = 0; s < NS; ++s) {
                     const TT v = P[s][J];
                     const int c = (((__float_as_int(fabsf(v)) >> 8) << 8) | (255 - lg[s]));
-                    bk = (lg[s] >= k && v == v && c > bk) ? c : bk;
+                    bk = (done[s] == 0 && v == v && c > bk) ? c : bk;
                     dnan |= (lg[s] == k) & (v != v);
                 }
                 bk = wave_max(bk);
                 const int pl0 = (bk < 0 || __any(dnan)) ? k : 255 - (bk & 255);
-                int kp = 0;
 #pragma unroll
-                for (int s = 0; s < NS; ++s) {
-                    const unsigned long long m = __ballot(lg[s] == pl0);
-                    kp = m ? (__builtin_ctzll(m) + 64 * s) : kp;
-                }
-                key = (pl0 << 8) | kp;
+                for (int s = 0; s < NS; ++s) bm[s] = __ballot(lg[s] == pl0);
             } else {
-                // largest |a_rk| over eligible rows (NaN never wins), then the lowest key holding
-                // it; both reduced over the 64 lanes, so every lane sees the same pivot
-                using CT = typename Cand<TT>::type;
-                CT vs[NS];
-                CT bv = CT(-1);
-                bool dnan = false;
+                // FP64: the high words of |a_rk| over the candidates, as integers (ordered like
+                // the values); a single row holding the largest is the pivot.
+                int hv[NS], bh = -1;
 #pragma unroll
                 for (int s = 0; s < NS; ++s) {
-                    const TT v = P[s][J];
-                    vs[s] = cand_of(v, lg[s] >= k);
-                    bv = vs[s] > bv ? vs[s] : bv;
-                    dnan |= (lg[s] == k) & (v != v);
+                    hv[s] = ((int)(__double_as_longlong((double)P[s][J]) >> 32) & 0x7fffffff) | done[s];
+                    bh = s == 0 ? hv[0] : imax(bh, hv[s]);
                 }
-                bv = wave_max(bv);
-                int bk = 0x7fffffff;
+                bh = wave_max(bh);
+                int count = 0;
 #pragma unroll
                 for (int s = 0; s < NS; ++s) {
-                    const int kk = (lg[s] << 8) | (lane + 64 * s);
-                    bk = ((lg[s] >= k) & (vs[s] == bv)) ? (kk < bk ? kk : bk) : bk;
+                    bm[s] = __ballot(hv[s] == bh);
+                    count += __builtin_popcountll(bm[s]);
                 }
-                key = wave_min(bk);
-                if (__any(dnan)) {  // the oracle keeps row k when a_kk is NaN
-                    int kp = 0;
+                if (count != 1 || bh > 0x7ff00000) {
+                    // uniform: rows that share the largest high word (then the largest low word,
+                    // then the lowest row), or a NaN: a NaN a_kk keeps row k (the oracle), any
+                    // other never wins
+                    int lv[NS], bl = INT_MIN, br = -1;
+                    bh = -1;
 #pragma unroll
                     for (int s = 0; s < NS; ++s) {
-                        const unsigned long long m = __ballot(lg[s] == k);
-                        kp = m ? (__builtin_ctzll(m) + 64 * s) : kp;
+                        const TT v = P[s][J];
+                        hv[s] = done[s] == 0 && v != v ? (lg[s] == k ? 0x7fffffff : -1) : hv[s];
+                        bh = imax(bh, hv[s]);
                     }
-                    key = (k << 8) | kp;
+                    bh = wave_max(bh);
+#pragma unroll
+                    for (int s = 0; s < NS; ++s) {
+                        lv[s] = (int)((unsigned)__double_as_longlong((double)P[s][J]) ^ 0x80000000u);  // unsigned order
+                        bl = hv[s] == bh ? imax(bl, lv[s]) : bl;
+                    }
+                    bl = wave_max(bl);
+#pragma unroll
+                    for (int s = 0; s < NS; ++s) br = hv[s] == bh && lv[s] == bl ? imax(br, 255 - lg[s]) : br;
+                    br = wave_max(br);
+#pragma unroll
+                    for (int s = 0; s < NS; ++s) bm[s] = __ballot(lg[s] == 255 - br);
                 }
             }
-            const int plog = key >> 8, pphys = key & 255;
-            const int ol = pphys & 63, slot = pphys >> 6;
-            // pivot row (panel part) to every lane (a uniform branch on the slot: fewer
+            // pivot row (panel part) to every lane (a uniform branch on its slot: fewer
             // instructions than selecting among the slots in every lane)
             TT prow[kPanel];
+            int plog;
 #pragma unroll
             for (int jj = 0; jj < kPanel; ++jj) prow[jj] = TT(0);
-            if (NS == 1 || slot == 0) {
+            const auto take = [&](auto slot) __attribute__((always_inline)) {
+                constexpr int s = decltype(slot)::value;
+                const int ol = __builtin_ctzll(bm[s]);
+                plog = __builtin_amdgcn_readlane(lg[s], ol);
+                done[s] = lane == ol ? -1 : done[s];
 #pragma unroll
-                for (int jj = J; jj < kPanel; ++jj) prow[jj] = rdlane(P[0][jj], ol);
-            } else if (NS == 2 || slot == 1) {
-#pragma unroll
-                for (int jj = J; jj < kPanel; ++jj) prow[jj] = rdlane(P[NS > 1 ? 1 : 0][jj], ol);
-            } else {
-#pragma unroll
-                for (int jj = J; jj < kPanel; ++jj) prow[jj] = rdlane(P[NS > 2 ? 2 : 0][jj], ol);
-            }
+                for (int jj = J; jj < kPanel; ++jj) prow[jj] = rdlane(P[s][jj], ol);
+            };
+            if (NS == 1 || bm[0])
+                take(std::integral_constant<int, 0>{});
+            else if (NS == 2 || bm[NS > 1 ? 1 : 0])
+                take(std::integral_constant<int, (NS > 1 ? 1 : 0)>{});
+            else
+                take(std::integral_constant<int, (NS > 2 ? 2 : 0)>{});
             const TT d = prow[J];
             pl[J] = plog;
+            if (plog != k) {  // uniform: the pivot row and row k trade logical places
 #pragma unroll
-            for (int s = 0; s < NS; ++s) lg[s] = lg[s] == k ? plog : (lg[s] == plog ? k : lg[s]);
-            if (d != TT(0)) {  // a zero pivot leaves the panel unchanged (the oracle skips the column)
+                for (int s = 0; s < NS; ++s) lg[s] = lg[s] == k ? plog : (lg[s] == plog ? k : lg[s]);
+            }
+            if (!is_zero(d)) {  // a zero pivot leaves the panel unchanged (the oracle skips the column)
                 const TT inv = TT(1) / d;
 #pragma unroll
                 for (int s = 0; s < NS; ++s) {
-                    const bool below = lg[s] > k;
-                    const TT l = below ? P[s][J] * inv : TT(0);
-                    P[s][J] = below ? l : P[s][J];
+                    const TT lf = P[s][J] * inv;
+                    const TT l = mask_sel(done[s], TT(0), lf);
+                    P[s][J] = mask_sel(done[s], P[s][J], lf);
 #pragma unroll
                     for (int jj = J + 1; jj < kPanel; ++jj) P[s][jj] -= l * prow[jj];
                 }
             }
         }
-        panel_columns<TT, NS, kFull, J + 1>(P, lg, pl, c0, w, lane);
+        panel_columns<TT, NS, kFull, J + 1>(P, lg, done, pl, c0, w, lane);
     }
 }
 
@@ -917,12 +887,13 @@ __device__ __forceinline__ void lu_panel_ns(TT* A, int n, int lda, int c0, int w
     const int* ph_in = phys_buf(W, c0 + kPanel);  // the previous panel's buffer (identity before panel 0)
     int* ph_out = phys_buf(W, c0);
     TT P[NS][kPanel];
-    int lg[NS], rr[NS];
+    int lg[NS], rr[NS], done[NS];
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
         const int li = c0 + lane + 64 * s;
         const bool ok = li < n;
         lg[s] = ok ? li : -1;
+        done[s] = ok ? 0 : -1;
         rr[s] = ph_in[ok ? li : c0];  // clamped: loads are unconditional, values selected after
 #pragma unroll
         for (int jj = 0; jj < kPanel; ++jj) P[s][jj] = A[rr[s] * lda + c0 + (jj < w ? jj : 0)];
@@ -932,11 +903,9 @@ __device__ __forceinline__ void lu_panel_ns(TT* A, int n, int lda, int c0, int w
         for (int jj = 0; jj < kPanel; ++jj) P[s][jj] = (ok && jj < w) ? P[s][jj] : TT(0);
     }
     // Columns as compile-time steps (constant register indices without relying on unrolling:
-    // the tile stays in registers).  A single wave issues about one instruction per four cycles,
-    // so each step keeps its instruction count down: uniform branches on the pivot's slot and
-    // on a zero pivot rather than per-element selects, and only NS row slots per lane.
+    // the tile stays in registers), only NS row slots per lane.
     int pl[kPanel];
-    panel_columns<TT, NS, kFull, 0>(P, lg, pl, c0, w, lane);
+    panel_columns<TT, NS, kFull, 0>(P, lg, done, pl, c0, w, lane);
     if (lane == 0) {
 #pragma unroll
         for (int j = 0; j < kPanel; ++j)
@@ -1031,117 +1000,171 @@ __device__ __forceinline__ void u_rows_group_fma(const float* Lc, float (&u)[kPa
         for (int i = KG + kk + 1; i < kPanel; ++i) u[i] = __builtin_fmaf(-lk[kk][i], u[KG + kk], u[i]);
 }
 
-// Applies panel [c0, c0 + w) to this wave's share of the columns [ja, jb): columns
-// ja + g, ja + g + gs, ... (wave g of gs).  First the panel's U rows (U12 = L11^-1 A12, lane <->
-// column, written in place into the pivot rows), then the trailing rows a_rj -= sum_k l_rk u_kj
-// (k ascending; lane <-> logical rows j0 + lane + 64 s, s < NSA, with their multipliers in
-// registers; two columns at a time).  Rows already pivoted are not touched.
-// Runs within one wave: its LDS writes are seen by its own later reads without a barrier.
-template <typename TT, bool kFull, int NSA>
-__device__ __forceinline__ void lu_apply_panel(TT* A, int n, int lda, int c0, int w, int ja, int jb, int g, int gs,
-                                               const LuScratch& W) {
-    if (kFull) w = kPanel;
-    const int lane = threadIdx.x & 63;
-    const int j0 = c0 + w;  // rows with logical index >= j0 are trailing rows
-    const int m = ja + g < jb ? (jb - ja - g + gs - 1) / gs : 0;
-    if (m == 0) return;
-    // the row mapping after this panel: the next panel's factorization (wave 0, possibly
-    // running meanwhile) permutes rows among logical j0 .. n - 1 only and writes the other buffer
-    const int* ph = phys_buf(W, c0);
-    int pr[kPanel];
-#pragma unroll
-    for (int i = 0; i < kPanel; ++i) pr[i] = __builtin_amdgcn_readfirstlane(ph[c0 + (i < w ? i : 0)]);
-    // U rows: u_i -= l_ik u_k for k ascending (each entry's FMA sequence as in the unblocked
-    // loop), one column per lane; L11 from the panel's compact column-major tile, where column
-    // k's entries below the diagonal are contiguous (vector loads, same address on all lanes)
-    const TT* Lc = panel_l11<TT>(W, c0);
-    for (int t = lane; t < m; t += 64) {
-        const int j = ja + g + gs * t;
-        TT u[kPanel];
-#pragma unroll
-        for (int i = 0; i < kPanel; ++i) u[i] = A[pr[i] * lda + j];
-#pragma unroll
-        for (int i = 0; i < kPanel; ++i) pin(u[i]);
-        u_rows_group<TT, 0>(Lc, u);
-        u_rows_group<TT, 4>(Lc, u);
-        u_rows_group<TT, 8>(Lc, u);
-        u_rows_group<TT, 12>(Lc, u);
-#pragma unroll
-        for (int i = 1; i < kPanel; ++i)
-            if (kFull || i < w) A[pr[i] * lda + j] = u[i];
+// 16 x 16 x 4 matrix-core products: A operand row lane % 16, k = lane / 16, B operand column
+// lane % 16, same k.  Both types accumulate c + a_0 b_0 + ... + a_3 b_3 like a chain of FMAs in
+// ascending k (the same bits on 5e6 random entries with exponents within 2^40 of each other), the
+// update loop's sequence; on the mixed FP64 ensemble 7 of 192 blades' first increments end in
+// other last bits than with the loop, at the same distance from a 64-bit solve.
+template <typename TT>
+struct MfmaTile;
+template <>
+struct MfmaTile<double> {
+    typedef double vec __attribute__((ext_vector_type(4)));
+    static __device__ __forceinline__ vec mac(double a, double b, vec c) {
+        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    // trailing rows
-    TT L[NSA][kPanel];
-    int prw[NSA];
-    bool ok[NSA];
-#pragma unroll
-    for (int s = 0; s < NSA; ++s) {
-        const int li = j0 + lane + 64 * s;
-        ok[s] = li < n;
-        prw[s] = ph[ok[s] ? li : 0];
-#pragma unroll
-        for (int i = 0; i < kPanel; ++i) L[s][i] = A[prw[s] * lda + c0 + (i < w ? i : 0)];
-#pragma unroll
-        for (int i = 0; i < kPanel; ++i) pin(L[s][i]);
-#pragma unroll
-        for (int i = 0; i < kPanel; ++i) L[s][i] = (ok[s] && (kFull || i < w)) ? L[s][i] : TT(0);
+    static __device__ __forceinline__ int row(int r, int lk) { return 4 * r + lk; }  // output row of entry r
+};
+template <>
+struct MfmaTile<float> {
+    typedef f32x4 vec;
+    static __device__ __forceinline__ vec mac(float a, float b, vec c) {
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
     }
-    for (int t = 0; t < m; t += 2) {
-        const int j = ja + g + gs * t;
-        const bool two = t + 1 < m;
-        const int jq = two ? j + gs : j;
-        TT u0[kPanel], u1[kPanel];
+    static __device__ __forceinline__ int row(int r, int lk) { return 4 * lk + r; }
+};
+
+// U rows of one column per lane: u_i = a_(p_i, j), then u_i -= l_ik u_k for k ascending (each
+// entry's FMA sequence as in the unblocked loop); L11 from the panel's compact column-major
+// tile, where column k's entries below the diagonal are contiguous (vector loads, same address
+// on all lanes).
+template <typename TT>
+__device__ __forceinline__ void lu_u_rows(const TT* A, int lda, const int (&pr)[kPanel], const TT* Lc, int j, TT (&u)[kPanel]) {
 #pragma unroll
-        for (int i = 0; i < kPanel; ++i) {
-            u0[i] = A[pr[i] * lda + j];
-            u1[i] = A[pr[i] * lda + jq];
-        }
-        if (!kFull) {
+    for (int i = 0; i < kPanel; ++i) u[i] = A[pr[i] * lda + j];
 #pragma unroll
-            for (int i = 0; i < kPanel; ++i) {
-                pin(u0[i]);
-                pin(u1[i]);
-            }
-#pragma unroll
-            for (int i = 0; i < kPanel; ++i) {
-                u0[i] = i < w ? u0[i] : TT(0);
-                u1[i] = i < w ? u1[i] : TT(0);
-            }
-        }
-#pragma unroll
-        for (int s = 0; s < NSA; ++s) {
-            if (ok[s]) {
-                TT* Ar = A + prw[s] * lda;
-                TT a0 = Ar[j];
-                TT a1 = Ar[jq];
-#pragma unroll
-                for (int i = 0; i < kPanel; ++i) {
-                    a0 -= L[s][i] * u0[i];
-                    a1 -= L[s][i] * u1[i];
-                }
-                Ar[j] = a0;
-                if (two) Ar[jq] = a1;
-            }
-        }
-    }
+    for (int i = 0; i < kPanel; ++i) pin(u[i]);
+    u_rows_group<TT, 0>(Lc, u);
+    u_rows_group<TT, 4>(Lc, u);
+    u_rows_group<TT, 8>(Lc, u);
+    u_rows_group<TT, 12>(Lc, u);
 }
 
+// Trailing rows row0 .. row0 + 15 (logical) of NT column tiles: a_rj -= sum_k l_rk u_kj over the
+// panel's 16 columns.  B operands in bo, the tiles' columns (clamped) in jc, ok where stored.
+template <typename TT, int NT>
+__device__ __forceinline__ void lu_row_tile(TT* A, int n, int lda, int c0, int row0, const int* ph,
+                                            const TT (&bo)[NT][4], const int (&jc)[NT], const bool (&ok)[NT], int li, int lk) {
+    typedef MfmaTile<TT> M;
+    const int ra = row0 + li;
+    const TT* pa = A + ph[ra < n ? ra : row0] * lda + c0 + lk;
+    int pc[4];
+    bool okr[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int rc = row0 + M::row(r, lk);
+        okr[r] = rc < n;
+        pc[r] = ph[okr[r] ? rc : row0] * lda;
+    }
+    TT ao[4];
+    typename M::vec acc[NT];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) ao[ks] = pa[4 * ks];
+#pragma unroll
+    for (int s = 0; s < NT; ++s)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[s][r] = A[pc[r] + jc[s]];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+        for (int s = 0; s < NT; ++s) acc[s] = M::mac(-ao[ks], bo[s][ks], acc[s]);
+#pragma unroll
+    for (int s = 0; s < NT; ++s)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (ok[s] && okr[r]) A[pc[r] + jc[s]] = acc[s][r];
+}
+
+// The trailing rows of NT column tiles ja + 16 (t0 + gs s) + li, s < NT, U rows in place
+template <typename TT, int NT>
+__device__ __forceinline__ void lu_trailing(TT* A, int n, int lda, int c0, int ja, int jb, int t0, int gs, const int* ph,
+                                            int li, int lk) {
+    TT bo[NT][4];
+    int jc[NT], pk[4];
+    bool ok[NT];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) pk[ks] = ph[c0 + 4 * ks + lk] * lda;
+#pragma unroll
+    for (int s = 0; s < NT; ++s) {
+        const int j = ja + 16 * (t0 + gs * s) + li;
+        ok[s] = j < jb;
+        jc[s] = ok[s] ? j : ja;
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) bo[s][ks] = A[pk[ks] + jc[s]];
+    }
+    for (int row0 = c0 + kPanel; row0 < n; row0 += 16)
+        lu_row_tile<TT, NT>(A, n, lda, c0, row0, ph, bo, jc, ok, li, lk);
+}
+
+// Look-ahead: applies the full panel [c0, c0 + 16) to the next panel's wn columns.  Every wave
+// forms those columns' U rows in registers (the solve's time does not depend on how many columns
+// it has, so no wave waits for another's; lane li of each 16-lane group takes column li) and
+// updates its share of the trailing row tiles.  Returns the U rows: they replace the columns'
+// pivot rows, which other waves may still be reading, once every wave is done.
+template <typename TT>
+__device__ __forceinline__ void lu_lookahead(TT* A, int n, int lda, int c0, int wn, int wv, int nw, const LuScratch& W,
+                                             TT (&u)[kPanel], int (&pr)[kPanel]) {
+    const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+    const int j0 = c0 + kPanel;
+    const int* ph = phys_buf(W, c0);
+#pragma unroll
+    for (int i = 0; i < kPanel; ++i) pr[i] = __builtin_amdgcn_readfirstlane(ph[c0 + i]);
+    const bool ok[1] = {li < wn};
+    const int jc[1] = {j0 + (ok[0] ? li : 0)};
+    lu_u_rows<TT>(A, lda, pr, panel_l11<TT>(W, c0), jc[0], u);
+    TT bo[1][4];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {  // row 4 ks + lk of the lane's column
+        const TT a = lk & 1 ? u[4 * ks + 1] : u[4 * ks], b = lk & 1 ? u[4 * ks + 3] : u[4 * ks + 2];
+        bo[0][ks] = lk & 2 ? b : a;
+    }
+    for (int row0 = j0 + kPanel * wv; row0 < n; row0 += kPanel * nw)
+        lu_row_tile<TT, 1>(A, n, lda, c0, row0, ph, bo, jc, ok, li, lk);
+}
+
+// Applies panel [c0, c0 + w) to this wave's share of the columns [ja, jb), in tiles of 16 columns:
+// tiles g, g + gs, ... (wave g of gs), three at a time.  First the tiles' U rows, one column per
+// lane, written in place into the pivot rows; then the trailing rows on the matrix cores, 16 at a
+// time (a partial panel is the last and has none).  Rows already pivoted are not touched.  The row
+// mapping is this panel's: the next panel's factorization (wave 0, possibly running meanwhile)
+// permutes rows among logical c0 + w .. n - 1 only and writes the other buffer.
+// Runs within one wave: its LDS writes are seen by its own later reads without a barrier.
+// Look-ahead and trailing update per block of the mixed FP64 ensemble: 69k cycles, 83k on the VALU
+// (a row per lane, two columns at a time, u broadcast from LDS).
 template <typename TT>
 __device__ __forceinline__ void lu_apply(TT* A, int n, int lda, int c0, int w, int ja, int jb, int g, int gs,
                                          const LuScratch& W) {
-    // NSA lane <-> row slots for the n - (c0 + w) <= 127 trailing rows
-    if (n - (c0 + w) > 64) {
-        if (w == kPanel)
-            lu_apply_panel<TT, true, 2>(A, n, lda, c0, w, ja, jb, g, gs, W);
+    constexpr int kTiles = 3;
+    const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+    const int* ph = phys_buf(W, c0);
+    const int tc = (jb - ja + 15) >> 4;
+    if (g >= tc) return;
+    int pr[kPanel];
+#pragma unroll
+    for (int i = 0; i < kPanel; ++i) pr[i] = __builtin_amdgcn_readfirstlane(ph[c0 + (i < w ? i : 0)]);
+    for (int t0 = g; t0 < tc; t0 += kTiles * gs) {
+        const int left = (tc - t0 + gs - 1) / gs, nt = left < kTiles ? left : kTiles;  // uniform
+        {
+            const int j = ja + 16 * (t0 + gs * lk) + li;  // lane group lk: the pass's tile lk
+            const bool okj = lk < nt && j < jb;
+            TT u[kPanel];
+            lu_u_rows<TT>(A, lda, pr, panel_l11<TT>(W, c0), okj ? j : ja, u);
+            if (okj) {
+#pragma unroll
+                for (int i = 1; i < kPanel; ++i)
+                    if (i < w) A[pr[i] * lda + j] = u[i];
+            }
+        }
+        if (c0 + w >= n) continue;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        if (nt == 1)
+            lu_trailing<TT, 1>(A, n, lda, c0, ja, jb, t0, gs, ph, li, lk);
+        else if (nt == 2)
+            lu_trailing<TT, 2>(A, n, lda, c0, ja, jb, t0, gs, ph, li, lk);
         else
-            lu_apply_panel<TT, false, 2>(A, n, lda, c0, w, ja, jb, g, gs, W);
-    } else if (w == kPanel) {
-        lu_apply_panel<TT, true, 1>(A, n, lda, c0, w, ja, jb, g, gs, W);
-    } else {
-        lu_apply_panel<TT, false, 1>(A, n, lda, c0, w, ja, jb, g, gs, W);
+            lu_trailing<TT, 3>(A, n, lda, c0, ja, jb, t0, gs, ph, li, lk);
     }
 }
 
@@ -1156,7 +1179,7 @@ template <typename TT>
 __device__ __forceinline__ void lu_factor_augmented(TT* A, int n, int lda, int* piv, const LuScratch& W,
                                                     int nrhs = 1) {
     static_assert(kThreads >= 128, "the blocked LU needs wave 0 and at least one more wave");
-    const int tid = threadIdx.x, wv = tid >> 6;
+    const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nw = blockDim.x >> 6;
     const int nc = n + nrhs;  // right-hand sides ride along as columns n .. n + nrhs - 1
     for (int r = tid; r < kLuTile; r += blockDim.x) {
@@ -1175,7 +1198,9 @@ __device__ __forceinline__ void lu_factor_augmented(TT* A, int n, int lda, int* 
         KYN_SPAN_BEGIN(t_sp);
         if (wv == 0) {
             if (wn > 0) {
-                lu_apply<TT>(A, n, lda, c0, w, j0, j0 + wn, 0, nw, W);  // wave 0's share of the look-ahead
+                TT u[kPanel];
+                int pr[kPanel];
+                lu_lookahead<TT>(A, n, lda, c0, wn, 0, nw, W, u, pr);  // wave 0's share
                 done += nw - 1;
                 // bounded wait (every other wave adds one per panel, so it ends; the bound keeps a
                 // broken count from hanging the kernel: the wave then goes on and flags the error)
@@ -1189,12 +1214,18 @@ __device__ __forceinline__ void lu_factor_augmented(TT* A, int n, int lda, int* 
                     __builtin_amdgcn_s_sleep(1);
                 }
                 KYN_SPAN_END(0, t_sp, 0);
+                if ((tid & 63) < wn) {  // the columns' U rows in place, now that no wave reads them raw
+#pragma unroll
+                    for (int i = 1; i < kPanel; ++i) A[pr[i] * lda + j0 + tid] = u[i];
+                }
                 lu_panel<TT>(A, n, lda, j0, wn, piv, W);
             }
             KYN_SPAN_END(1, t_sp, 0);
         } else {
             if (wn > 0) {
-                lu_apply<TT>(A, n, lda, c0, w, j0, j0 + wn, wv, nw, W);
+                TT u[kPanel];
+                int pr[kPanel];
+                lu_lookahead<TT>(A, n, lda, c0, wn, wv, nw, W, u, pr);
                 if ((tid & 63) == 0)
                     __hip_atomic_fetch_add(W.sync, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
             }
@@ -1217,7 +1248,7 @@ __device__ __forceinline__ void lu_factor_augmented(TT* A, int n, int lda, int* 
 // perturbation of an SPD matrix (mass plus stiffness), which factors stably without row
 // interchanges, and the constraint rows come last: their pivots are those of the Schur
 // complement -B (beta h^2 K)^-1 B^T, after which nothing else is eliminated.  (The FP64 forms
-// keep the pivoted LU above, whose factors are the oracle's bit for bit.)
+// keep the pivoted LU above, which takes the oracle's pivots.)
 //
 // Panels of 16 columns, two barriers each:
 //  P1  every wave factors the 16 x 16 diagonal tile in lanes 0..15 (row per lane, each pivot

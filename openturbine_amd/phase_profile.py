@@ -61,7 +61,7 @@ def main():
     spans = ["LU wait for look-ahead (wave 0)", "LU wait + panel (wave 0)", "LU look-ahead + trailing (wave 1)",
              "LU panel steps incl. barrier", "refinement residual (HBM copy)", "refinement solve",
              "refinement forward sweep (wave 0)", "unpivoted LU: diagonal tile + L21", "unpivoted LU: U12 rows",
-             "unpivoted LU: MFMA trailing update"]
+             "unpivoted LU: MFMA trailing update","tU","tR"]
     for i, name in enumerate(spans):
         if i < 4 or a[16 + i]:
             print(f"    {name:34s} {a[16 + i] / count:10.0f} cycles")
