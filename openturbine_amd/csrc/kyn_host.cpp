@@ -49,6 +49,8 @@ void launch_cond_backsub(const DevSys& S, double* xout, hipStream_t st);
 void launch_cond_scatter_z(const DevSys& S, int b, int nz, double* xout, hipStream_t st);
 void launch_block_axpy_copy(const DevSys& S, int b, int n, const double* d, double* x, double* r, hipStream_t st);
 void launch_f64_to_f32(const double* x, float* y, size_t count, hipStream_t st);
+size_t state_copy_doubles(const DevSys& S);
+void launch_state_copy(const DevSys& S, double* saved, bool restore, hipStream_t st);
 void launch_pack_motion(const DevSys& S, double* out, hipStream_t st);
 void launch_add_f32_to_f64(const float* d, double* x, int count, hipStream_t st);
 void launch_plain_epilogue(const DevSys& S, hipStream_t st);
@@ -205,10 +207,15 @@ struct Arena {
         return d;
     }
     template <typename T>
-    T* zeros(size_t n) {
+    T* alloc(size_t n) {  // not cleared
         T* d = nullptr;
         hip_check(hipMalloc(&d, std::max<size_t>(n, 1) * sizeof(T)), "hipMalloc");
         ptrs.push_back(d);
+        return d;
+    }
+    template <typename T>
+    T* zeros(size_t n) {
+        T* d = alloc<T>(n);
         hip_check(hipMemset(d, 0, std::max<size_t>(n, 1) * sizeof(T)), "hipMemset");
         return d;
     }
@@ -241,8 +248,7 @@ struct kyn_system_s {
     std::vector<int> node_block, node_local;
     std::vector<int> con_local, con_rows, con_model_row, con_block;
     std::vector<std::vector<int>> model_gdof_to_block_vec;  // per model: global dof -> rhs index
-    // saved state (CopyStateData)
-    std::vector<double> saved;
+    double* saved{};  // saved state (CopyStateData), on the device; allocated on first use
     bool has_saved{false};
     // large blocks (library LU): block ids, sizes, matrix offsets, pivots, scratch vectors
     std::vector<int> large_blocks, large_n, large_nsys;
@@ -2105,19 +2111,10 @@ int kyn_model_get_beam_element(kyn_model m, size_t elem, size_t* node_ids, doubl
 int kyn_save_state(kyn_system s) {
     return guarded([&] {
         if (!s) throw KynError(KYN_ERR_INVALID, "null system");
-        const size_t n = s->num_nodes;
-        s->saved.assign(n * (7 * 3 + 6 * 5) + 1, 0.);
-        double* o = s->saved.data();
-        const int fields[] = {KYN_X, KYN_Q_DELTA, KYN_Q_PREV, KYN_Q, KYN_V, KYN_VD, KYN_A, KYN_F};
-        for (int f : fields) {
-            int w = 0;
-            double* p = field_ptr(s, f, w);
-            hip_check(hipMemcpy(o, p, n * w * sizeof(double), hipMemcpyDeviceToHost), "D2H");
-            o += n * w;
-        }
-        int slot = 0;
-        hip_check(hipMemcpy(&slot, s->S.sched_slot, sizeof(int), hipMemcpyDeviceToHost), "D2H");
-        *o = static_cast<double>(slot);
+        if (!s->saved) s->saved = s->arena.alloc<double>(kyn::state_copy_doubles(s->S));
+        kyn::launch_state_copy(s->S, s->saved, false, s->stream);
+        hip_check(hipGetLastError(), "k_state_copy launch");
+        hip_check(hipStreamSynchronize(s->stream), "sync");
         s->has_saved = true;
         return KYN_OK;
     });
@@ -2125,17 +2122,9 @@ int kyn_save_state(kyn_system s) {
 int kyn_restore_state(kyn_system s) {
     return guarded([&] {
         if (!s || !s->has_saved) throw KynError(KYN_ERR_INVALID, "no saved state");
-        const size_t n = s->num_nodes;
-        const double* o = s->saved.data();
-        const int fields[] = {KYN_X, KYN_Q_DELTA, KYN_Q_PREV, KYN_Q, KYN_V, KYN_VD, KYN_A, KYN_F};
-        for (int f : fields) {
-            int w = 0;
-            double* p = field_ptr(s, f, w);
-            hip_check(hipMemcpy(p, o, n * w * sizeof(double), hipMemcpyHostToDevice), "H2D");
-            o += n * w;
-        }
-        const int slot = static_cast<int>(*o);
-        hip_check(hipMemcpy(s->S.sched_slot, &slot, sizeof(int), hipMemcpyHostToDevice), "H2D");
+        kyn::launch_state_copy(s->S, s->saved, true, s->stream);
+        hip_check(hipGetLastError(), "k_state_copy launch");
+        hip_check(hipStreamSynchronize(s->stream), "sync");
         return KYN_OK;
     });
 }

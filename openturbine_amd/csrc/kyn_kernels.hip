@@ -3309,6 +3309,52 @@ __global__ void k_pack_motion(DevSys S, double* out) {
     }
 }
 
+// CopyStateData (copy_state_data.hpp:20-34) to and from the saved state, in one launch: field
+// blockIdx.y of x, q_delta, q_prev, q, v, vd, a, f (each padded to whole 16-byte pairs in the saved
+// buffer), and the schedule row.  Bound by HBM: two doubles per lane and access.  The state of 4096
+// rotors (67 MB) took 7 ms to restore from host memory, a copy per field.
+__host__ __device__ inline size_t state_field_pairs(size_t nodes, int width) { return (nodes * width + 1) / 2; }
+__global__ void __launch_bounds__(256) k_state_copy(DevSys S, double* saved, int restore) {
+    double* const fields[8] = {S.x, S.q_delta, S.q_prev, S.q, S.v, S.vd, S.a, S.f};
+    constexpr int width[8] = {7, 6, 7, 7, 6, 6, 6, 6};
+    const size_t n = S.num_nodes;
+    const int f = blockIdx.y;
+    double* live = nullptr;
+    size_t off = 0, count = 0;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        if (k < f) off += 2 * state_field_pairs(n, width[k]);
+        if (k == f) {
+            live = fields[k];
+            count = n * width[k];
+        }
+    }
+    const double* src = restore ? saved + off : live;
+    double* dst = restore ? live : saved + off;
+    const size_t step = (size_t)gridDim.x * blockDim.x, i0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const double2* src2 = reinterpret_cast<const double2*>(src);
+    double2* dst2 = reinterpret_cast<double2*>(dst);
+    for (size_t i = i0; i < count / 2; i += step) dst2[i] = src2[i];
+    if (i0 == 0) {
+        if (count & 1) dst[count - 1] = src[count - 1];
+        if (f == 0) {
+            double* slot = saved + 2 * (5 * state_field_pairs(n, 6) + 3 * state_field_pairs(n, 7));
+            if (restore)
+                *S.sched_slot = (int)*slot;
+            else
+                *slot = (double)*S.sched_slot;
+        }
+    }
+}
+size_t state_copy_doubles(const DevSys& S) {
+    return 2 * (5 * state_field_pairs(S.num_nodes, 6) + 3 * state_field_pairs(S.num_nodes, 7)) + 1;
+}
+void launch_state_copy(const DevSys& S, double* saved, bool restore, hipStream_t st) {
+    const size_t pairs = state_field_pairs(S.num_nodes, 7);
+    const unsigned blocks = (unsigned)(pairs < 256 * 256 ? (pairs + 255) / 256 : 256);
+    hipLaunchKernelGGL(k_state_copy, dim3(blocks > 0 ? blocks : 1, 8), dim3(256), 0, st, S, saved, restore ? 1 : 0);
+}
+
 // mixed precision helpers for the large-block refinement
 __global__ void k_f64_to_f32(const double* x, float* y, size_t count) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
