@@ -45,8 +45,7 @@ size_t cond_lds(int ne, int me);
 void launch_cond_factor(const DevSys& S, size_t lds, bool fp32, const double* rin, hipStream_t st);
 void launch_cond_interface(const DevSys& S, int b, int nz, const int* colour_sizes, int ncolour, const double* rin,
                            hipStream_t st);
-void launch_cond_backsub(const DevSys& S, double* xout, hipStream_t st);
-void launch_cond_scatter_z(const DevSys& S, int b, int nz, double* xout, hipStream_t st);
+void launch_cond_backsub(const DevSys& S, double* xout, bool uncondition, hipStream_t st);
 void launch_block_axpy_copy(const DevSys& S, int b, int n, const double* d, double* x, double* r, hipStream_t st);
 void launch_f64_to_f32(const double* x, float* y, size_t count, hipStream_t st);
 size_t state_copy_doubles(const DevSys& S);
@@ -885,6 +884,7 @@ void solve_large_blocks(kyn_system_s* s) {
     // (each re-runs the condensed solve on the FP64 residual r = b - A x).
     if (S.num_cond_elems > 0) {
         const bool fp32 = S.precision != KYN_TANGENT_FP64;
+        const bool refined = fp32 && S.refine_sweeps > 0;
         auto cond_solve = [&](const double* rin, double* xout) {
             kyn::launch_cond_factor(S, s->cond_lds_bytes, fp32, rin, st);
             hip_check(hipGetLastError(), "k_cond_factor launch");
@@ -904,17 +904,10 @@ void solve_large_blocks(kyn_system_s* s) {
                 blas_check(rocsolver_dgetrs(s->blas, rocblas_operation_none, nz, 1, Z, nz, s->ipiv, z, nz),
                            "rocsolver_dgetrs");
             }
-            kyn::launch_cond_backsub(S, xout, st);
-            for (size_t k = 0; k < s->large_blocks.size(); ++k) {
-                const int b = s->large_blocks[k];
-                if (!s->large_cond[k] || !s->model_active_host[s->block_model[b]]) continue;
-                kyn::launch_cond_scatter_z(S, b, s->large_nz[k], xout, st);
-            }
+            kyn::launch_cond_backsub(S, xout, !refined, st);
         };
-        if (!fp32) {
-            cond_solve(S.rhs, S.xsol);
-        } else {
-            cond_solve(S.rhs, S.xsol);
+        cond_solve(S.rhs, S.xsol);
+        if (refined) {
             for (int sweep = 0; sweep < S.refine_sweeps; ++sweep) {
                 for (size_t k = 0; k < s->large_blocks.size(); ++k) {
                     const int b = s->large_blocks[k], n = s->large_n[k];
@@ -930,7 +923,7 @@ void solve_large_blocks(kyn_system_s* s) {
                 }
             }
         }
-        for (size_t k = 0; k < s->large_blocks.size(); ++k) {
+        for (size_t k = 0; refined && k < s->large_blocks.size(); ++k) {
             const int b = s->large_blocks[k];
             if (!s->large_cond[k] || !s->model_active_host[s->block_model[b]]) continue;
             kyn::launch_large_uncondition(S, b, s->large_n[k], st);
@@ -1180,6 +1173,7 @@ kyn_system kyn_system_create(const kyn_model* models, size_t num_models, const k
         // ---- sizes and eligibility
         S.num_models = static_cast<int>(num_models);
         S.num_blocks = static_cast<int>(B.block_n.size());
+        for (int bn : B.block_n) S.num_small_blocks += bn <= kyn::kMaxBlockDofs ? 1 : 0;
         S.num_elems = static_cast<int>(B.elem_N.size());
         S.num_nodes = static_cast<int>(B.node_block.size());
         S.num_cons = static_cast<int>(B.con_type.size());

@@ -2101,35 +2101,60 @@ __device__ __forceinline__ double block_error_and_update(const DevSys& S, int b,
         __syncthreads();
         return sum;
     }
-    for (int i = t; i < n; i += blockDim.x) {
-        double e;
-        if (i < nsys) {
-            const int node = S.block_nodes[nb0 + i / 6];
-            const double xi = S.q_delta[node * 6 + i % 6] * p.h;
-            e = xs[i] / (p.atol + p.rtol * fabs(xi));
-        } else {
-            // constraint row: find constraint by local row
-            e = 0.;
-            for (int k = S.block_con_begin[b]; k < S.block_con_end[b]; ++k) {
-                const int c = S.block_cons[k];
-                const int r = i - S.con_local[c];
-                if (r >= 0 && r < S.con_rows[c]) {
-                    e = xs[i] / (p.atol + p.rtol * fabs(S.con_lambda[c * 6 + r]));
-                }
-            }
+    // a large block (one workgroup of 1024, plain form): bound by the dependent loads block_nodes ->
+    // state, so four rows' are in flight per thread, and constraint rows go by constraint (searching
+    // each row's constraint is a chain as long as the block has constraints).  8459 dofs, 66
+    // constraints: 79 us with 256 threads, a row at a time and the search; 23 us.
+    for (int i0 = t; i0 < nsys; i0 += 4 * blockDim.x) {
+        int k[4];
+        double qd[4], x[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int i = i0 + u * (int)blockDim.x < nsys ? i0 + u * (int)blockDim.x : i0;
+            k[u] = S.block_nodes[nb0 + i / 6] * 6 + i % 6;
+            x[u] = xs[i];
         }
-        term += e * e;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) qd[u] = S.q_delta[k[u]];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const double e = x[u] / (p.atol + p.rtol * fabs(qd[u] * p.h));
+            term += i0 + u * (int)blockDim.x < nsys ? e * e : 0.;
+        }
+    }
+    for (int q = S.block_con_begin[b] + t; q < S.block_con_end[b]; q += blockDim.x) {
+        const int c = S.block_cons[q], lr = S.con_local[c], rows = S.con_rows[c];
+        for (int r = 0; r < rows; ++r) {
+            const double e = xs[lr + r] / (p.atol + p.rtol * fabs(S.con_lambda[c * 6 + r]));
+            term += e * e;
+        }
     }
     const double sum = block_sum(term, red);
     // update (after every thread has read q_delta / lambda for the error)
-    for (int i = t; i < nsys; i += blockDim.x) {
-        const int node = S.block_nodes[nb0 + i / 6];
-        const int k = node * 6 + i % 6;
-        const double dx = xs[i];
-        S.q_delta[k] += dx / p.h;
-        if (p.is_dynamic) {
-            S.v[k] += p.gamma_prime * dx;
-            S.vd[k] += p.beta_prime * dx;
+    for (int i0 = t; i0 < nsys; i0 += 4 * blockDim.x) {
+        int k[4];
+        double dx[4], qd[4], v[4], vd[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int i = i0 + u * (int)blockDim.x < nsys ? i0 + u * (int)blockDim.x : i0;
+            k[u] = S.block_nodes[nb0 + i / 6] * 6 + i % 6;
+            dx[u] = xs[i];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            qd[u] = S.q_delta[k[u]];
+            v[u] = S.v[k[u]];
+            vd[u] = S.vd[k[u]];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            if (i0 + u * (int)blockDim.x < nsys) {
+                S.q_delta[k[u]] = qd[u] + dx[u] / p.h;
+                if (p.is_dynamic) {
+                    S.v[k[u]] = v[u] + p.gamma_prime * dx[u];
+                    S.vd[k[u]] = vd[u] + p.beta_prime * dx[u];
+                }
+            }
         }
     }
     for (int k = S.block_con_begin[b] + t; k < S.block_con_end[b]; k += blockDim.x) {
@@ -2442,10 +2467,6 @@ __global__ void __launch_bounds__(kThreads) k_plain_predict(DevSys S) {
     }
 }
 
-__global__ void k_plain_clear_flag(DevSys S) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) *S.any_active = 0;
-}
-
 // node -> model through the block table; nodes without dofs take no part in the iteration
 __device__ __forceinline__ int node_model(const DevSys& S, int node) {
     const int b = S.node_block[node];
@@ -2455,6 +2476,7 @@ __device__ __forceinline__ int node_model(const DevSys& S, int node) {
 // UpdateTangentOperator (src/step/update_tangent_operator.hpp:13-26)
 __global__ void k_plain_tangent(DevSys S) {
     const int node = blockIdx.x * blockDim.x + threadIdx.x;
+    if (node == 0) *S.any_active = 0;  // set again by this iteration's update
     if (node >= S.num_nodes) return;
     const int m = node_model(S, node);
     if (m < 0 || !S.model_active[m]) return;
@@ -3251,9 +3273,24 @@ __global__ void __launch_bounds__(kTreeThreads) k_tree_interface(DevSys S, int b
     }
 }
 
-// Element dofs from the interface solution: x_e = Y_b - Y_B lambda_e; interface rows copied
-__global__ void __launch_bounds__(kThreads) k_cond_backsub(DevSys S, double* xout) {
-    const int ce = blockIdx.x, t = threadIdx.x;
+// Element dofs from the interface solution: x_e = Y_b - Y_B lambda_e (a workgroup per element);
+// interface rows copied (a workgroup per block after those).  uncondition: multiplier rows divided
+// by the conditioner on the way (UnconditionSolution, where no refinement follows).
+__global__ void __launch_bounds__(kThreads) k_cond_backsub(DevSys S, double* xout, int uncondition) {
+    const int t = threadIdx.x;
+    if ((int)blockIdx.x >= S.num_cond_elems) {
+        const int b = blockIdx.x - S.num_cond_elems;
+        const int z0 = S.block_z_off[b], nz = S.block_z_off[b + 1] - z0;
+        if (nz == 0 || !S.model_active[S.block_model[b]]) return;
+        const int nsys = S.block_nsys[b];
+        for (int i = t; i < nz; i += blockDim.x) {
+            const int row = S.cond_z[z0 + i];
+            const double z = S.zrhs[z0 + i];
+            xout[S.block_vec_off[b] + row] = uncondition && row >= nsys ? z / S.p.conditioner : z;
+        }
+        return;
+    }
+    const int ce = blockIdx.x;
     const int b = S.cond_elem_block[ce];
     if (!S.model_active[S.block_model[b]]) return;
     const int r0 = S.cond_rows_off[ce], ne = S.cond_rows_off[ce + 1] - r0;
@@ -3268,12 +3305,6 @@ __global__ void __launch_bounds__(kThreads) k_cond_backsub(DevSys S, double* xou
         for (int k = 0; k < me; ++k) v -= Y[(size_t)k * ne + i] * z[lz[k]];
         x[rows[i]] = v;
     }
-}
-__global__ void k_cond_scatter_z(DevSys S, int b, double* xout) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int z0 = S.block_z_off[b], nz = S.block_z_off[b + 1] - z0;
-    if (i >= nz || !S.model_active[S.block_model[b]]) return;
-    xout[S.block_vec_off[b] + S.cond_z[z0 + i]] = S.zrhs[z0 + i];
 }
 // refinement bookkeeping of one block: x += d (x non-null), r = rhs (r non-null, before r -= A x)
 __global__ void k_block_axpy_copy(DevSys S, int b, const double* d, double* x, double* r) {
@@ -3366,7 +3397,8 @@ __global__ void k_add_f32_to_f64(const float* d, double* x, int count) {
 }
 
 // CalculateConvergenceError + UpdateStatePrediction + UpdateConstraintPrediction
-__global__ void __launch_bounds__(kThreads) k_plain_update(DevSys S, int iter) {
+// 256 threads per model, 1024 where a system has large blocks
+__global__ void __launch_bounds__(1024) k_plain_update(DevSys S, int iter) {
     __shared__ double red[16];
     const int m = blockIdx.x, t = threadIdx.x;
     if (!S.model_active[m]) return;
@@ -3482,8 +3514,7 @@ void launch_plain_predict(const DevSys& S, hipStream_t st) {
 void launch_plain_update(const DevSys& S, int iter, hipStream_t st);
 void launch_plain_iteration(const DevSys& S, int Nm, int Qm, int nm, int iter, bool solve,
                             hipStream_t st, hipEvent_t e0, hipEvent_t e1, bool defer_update) {
-    hipLaunchKernelGGL(k_plain_clear_flag, dim3(1), dim3(64), 0, st, S);
-    hipLaunchKernelGGL(k_plain_tangent, dim3((S.num_nodes + 255) / 256), dim3(256), 0, st, S);
+    hipLaunchKernelGGL(k_plain_tangent, dim3(S.num_nodes > 0 ? (S.num_nodes + 63) / 64 : 1), dim3(64), 0, st, S);
     if (e0) (void)hipEventRecord(e0, st);
     if (S.num_elems > 0) {
         if (S.precision)
@@ -3498,17 +3529,18 @@ void launch_plain_iteration(const DevSys& S, int Nm, int Qm, int nm, int iter, b
         hipLaunchKernelGGL(k_plain_points, dim3((S.num_masses + S.num_springs + 63) / 64), dim3(64), 0, st, S);
     if (S.num_cons > 0)
         hipLaunchKernelGGL(k_plain_constraints, dim3((S.num_cons + 63) / 64), dim3(64), 0, st, S);
-    hipLaunchKernelGGL(k_plain_assemble, dim3(S.num_blocks), dim3(kThreads), 0, st, S);
+    if (S.num_small_blocks > 0) hipLaunchKernelGGL(k_plain_assemble, dim3(S.num_blocks), dim3(kThreads), 0, st, S);
     if (S.num_big_items > 0) {
         hipLaunchKernelGGL(k_crs_zero, dim3(512), dim3(256), 0, st, S);
         hipLaunchKernelGGL(k_large_assemble, dim3(S.num_big_items), dim3(kThreads), 0, st, S);
     }
     if (!solve) return;
-    hipLaunchKernelGGL(k_plain_solve, dim3(S.num_blocks), dim3(kThreads), solve_lds_bytes(nm), st, S, nm);
+    if (S.num_small_blocks > 0)
+        hipLaunchKernelGGL(k_plain_solve, dim3(S.num_blocks), dim3(kThreads), solve_lds_bytes(nm), st, S, nm);
     if (!defer_update) launch_plain_update(S, iter, st);
 }
 void launch_plain_update(const DevSys& S, int iter, hipStream_t st) {
-    hipLaunchKernelGGL(k_plain_update, dim3(S.num_models), dim3(kThreads), 0, st, S, iter);
+    hipLaunchKernelGGL(k_plain_update, dim3(S.num_models), dim3(S.num_big_items > 0 ? 1024 : kThreads), 0, st, S, iter);
 }
 size_t cond_lds(int ne, int me) { return (size_t)cond_lds_bytes(ne, me); }
 void launch_cond_factor(const DevSys& S, size_t lds, bool fp32, const double* rin, hipStream_t st) {
@@ -3525,11 +3557,9 @@ void launch_cond_interface(const DevSys& S, int b, int nz, const int* colour_siz
     for (int col = 0; col < ncolour; ++col)
         hipLaunchKernelGGL(k_cond_interface, dim3((colour_sizes[col] * kStride + 255) / 256), dim3(256), 0, st, S, b, col);
 }
-void launch_cond_backsub(const DevSys& S, double* xout, hipStream_t st) {
-    hipLaunchKernelGGL(k_cond_backsub, dim3(S.num_cond_elems), dim3(kThreads), 0, st, S, xout);
-}
-void launch_cond_scatter_z(const DevSys& S, int b, int nz, double* xout, hipStream_t st) {
-    hipLaunchKernelGGL(k_cond_scatter_z, dim3((nz + 255) / 256), dim3(256), 0, st, S, b, xout);
+void launch_cond_backsub(const DevSys& S, double* xout, bool uncondition, hipStream_t st) {
+    hipLaunchKernelGGL(k_cond_backsub, dim3(S.num_cond_elems + S.num_blocks), dim3(kThreads), 0, st, S, xout,
+                       uncondition ? 1 : 0);
 }
 void launch_block_axpy_copy(const DevSys& S, int b, int n, const double* d, double* x, double* r, hipStream_t st) {
     hipLaunchKernelGGL(k_block_axpy_copy, dim3((n + 255) / 256), dim3(256), 0, st, S, b, d, x, r);

@@ -147,6 +147,7 @@ struct DevSys {
     unsigned contract_mfma_mask;      // FP32 tangent: bit N set -> element size N contracts on the
                                       // matrix cores, else on the VALU register tile
     const int* block_large;           // 1 if the block takes the large path
+    int num_small_blocks;             // blocks that do not
     const int64_t* crs_rp_off;        // per block: into crs_rp (n + 1 block-local row pointers)
     const int64_t* crs_nz_off;        // per block: into crs_col / crs_val
     const int* crs_rp;
