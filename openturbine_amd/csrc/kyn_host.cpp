@@ -43,6 +43,8 @@ void launch_crs_to_dense(const DevSys& S, int b, int n, hipStream_t st);
 void launch_tree_interface(const DevSys& S, int b, hipStream_t st);
 size_t cond_lds(int ne, int me);
 void launch_cond_factor(const DevSys& S, size_t lds, bool fp32, const double* rin, hipStream_t st);
+size_t cond_resolve_lds(int ne);
+void launch_cond_resolve(const DevSys& S, size_t lds, const double* rin, hipStream_t st);
 void launch_cond_interface(const DevSys& S, int b, int nz, const int* colour_sizes, int ncolour, const double* rin,
                            hipStream_t st);
 void launch_cond_backsub(const DevSys& S, double* xout, bool uncondition, hipStream_t st);
@@ -257,7 +259,7 @@ struct kyn_system_s {
     std::vector<int> tree_nvert;                  // per block: vertices of its interface tree (0: dense solve)
     std::vector<std::vector<int>> colour_sizes;   // per block: condensed elements of each colour
     std::vector<int64_t> large_Z_off;
-    size_t cond_lds_bytes{0};
+    size_t cond_lds_bytes{0}, cond_resolve_lds_bytes{0};
     rocblas_handle blas{};
     rocblas_int *ipiv{}, *info{};
     double *rvec{}, *bvec{};
@@ -881,13 +883,16 @@ void solve_large_blocks(kyn_system_s* s) {
     const hipStream_t st = s->stream;
     // condensed blocks: element eliminations (all elements at once), interface LU per block,
     // element back substitution.  FP32 option: element factors in FP32, FP64 refinement sweeps
-    // (each re-runs the condensed solve on the FP64 residual r = b - A x).
+    // (each a condensed solve with the same factors for the FP64 residual r = b - A x).
     if (S.num_cond_elems > 0) {
         const bool fp32 = S.precision != KYN_TANGENT_FP64;
         const bool refined = fp32 && S.refine_sweeps > 0;
-        auto cond_solve = [&](const double* rin, double* xout) {
-            kyn::launch_cond_factor(S, s->cond_lds_bytes, fp32, rin, st);
-            hip_check(hipGetLastError(), "k_cond_factor launch");
+        auto cond_solve = [&](const double* rin, double* xout, bool factor) {
+            if (factor)
+                kyn::launch_cond_factor(S, s->cond_lds_bytes, fp32, rin, st);
+            else
+                kyn::launch_cond_resolve(S, s->cond_resolve_lds_bytes, rin, st);
+            hip_check(hipGetLastError(), "condensed element solve launch");
             for (size_t k = 0; k < s->large_blocks.size(); ++k) {
                 const int b = s->large_blocks[k], nz = s->large_nz[k];
                 if (!s->large_cond[k] || !s->model_active_host[s->block_model[b]]) continue;
@@ -906,7 +911,7 @@ void solve_large_blocks(kyn_system_s* s) {
             }
             kyn::launch_cond_backsub(S, xout, !refined, st);
         };
-        cond_solve(S.rhs, S.xsol);
+        cond_solve(S.rhs, S.xsol, true);
         if (refined) {
             for (int sweep = 0; sweep < S.refine_sweeps; ++sweep) {
                 for (size_t k = 0; k < s->large_blocks.size(); ++k) {
@@ -915,7 +920,7 @@ void solve_large_blocks(kyn_system_s* s) {
                     // r = b - A x on the CRS matrix (FP64)
                     kyn::launch_crs_residual(S, b, n, S.xsol, s->rfull, st);
                 }
-                cond_solve(s->rfull, s->dfull);
+                cond_solve(s->rfull, s->dfull, false);
                 for (size_t k = 0; k < s->large_blocks.size(); ++k) {
                     const int b = s->large_blocks[k], n = s->large_n[k];
                     if (!s->large_cond[k] || !s->model_active_host[s->block_model[b]]) continue;
@@ -1571,6 +1576,17 @@ kyn_system kyn_system_create(const kyn_model* models, size_t num_models, const k
                 S.cond_S_off = Ar.up(S_off);
                 S.Ybuf = Ar.zeros<double>(static_cast<size_t>(Y_tot));
                 S.Sbuf = Ar.zeros<double>(static_cast<size_t>(S_tot));
+                if (S.precision != KYN_TANGENT_FP64 && S.refine_sweeps > 0) {  // the factors, for the sweeps
+                    std::vector<int64_t> fac_off(ce_elem.size() + 1, 0);
+                    for (size_t c = 0; c < ce_elem.size(); ++c) {
+                        const int ne = rows_off[c + 1] - rows_off[c];
+                        fac_off[c + 1] = fac_off[c] + static_cast<int64_t>(ne) * ne;
+                        sys->cond_resolve_lds_bytes = std::max(sys->cond_resolve_lds_bytes, kyn::cond_resolve_lds(ne));
+                    }
+                    S.cond_fac = Ar.zeros<float>(static_cast<size_t>(fac_off.back()));
+                    S.cond_fac_off = Ar.up(fac_off);
+                    S.cond_fac_row = Ar.zeros<int>(rows.size());
+                }
                 S.block_z_off = Ar.up(z_off);
                 S.cond_z = Ar.up(zl);
                 S.block_ce_begin = Ar.up(ce_begin);

@@ -2884,6 +2884,29 @@ __host__ __device__ inline int cond_lds_bytes(int ne, int me) {
     return align16(ne * lda * 8) + 2 * kLuTile * 4 + 2 * 256 * 8 + 16 + align16(ne * 4) + ne * (me + 1) * 8;
 }
 
+// Constraint row l (a cond_lam entry) of an element times an element vector y: four entries'
+// loads in flight, summed in order.
+__device__ __forceinline__ double cond_row_dot(const DevSys& S, const double* V, int l, const double* y) {
+    const int u0 = S.cond_bt_off[l], u1 = S.cond_bt_off[l + 1];
+    double acc = 0.;
+    for (int u = u0; u < u1; u += 4) {
+        int sq[4], cq[4];
+        double vq[4];
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            const int uu = u + w < u1 ? u + w : u;
+            sq[w] = S.cond_bt_src[uu];
+            cq[w] = S.cond_bt_col[uu];
+        }
+#pragma unroll
+        for (int w = 0; w < 4; ++w) vq[w] = V[sq[w]];
+#pragma unroll
+        for (int w = 0; w < 4; ++w)
+            if (u + w < u1) acc += vq[w] * y[cq[w]];
+    }
+    return acc;
+}
+
 // rin: right-hand side vector in the layout of S.rhs (the conditioned rhs, or a refinement
 // residual).  TT: storage type of the element factors (FP64, or FP32 with FP64 accumulation in
 // the triangular solves).
@@ -2946,25 +2969,63 @@ __device__ __forceinline__ void cond_factor_body(DevSys& S, const double* rin) {
     double* Sm = S.Sbuf + S.cond_S_off[ce];
     for (int q = t; q < me * nrhs; q += blockDim.x) {  // S_e = B_e Y: constraint row lam[k]'s entries in this element
         const int k = q % me, c = q / me;
-        const int u0 = S.cond_bt_off[l0 + k], u1 = S.cond_bt_off[l0 + k + 1];
-        double acc = 0.;
-        for (int u = u0; u < u1; u += 4) {  // four entries' loads in flight, summed in order
-            int sq[4], cq[4];
-            double vq[4];
-#pragma unroll
-            for (int w = 0; w < 4; ++w) {
-                const int uu = u + w < u1 ? u + w : u;
-                sq[w] = S.cond_bt_src[uu];
-                cq[w] = S.cond_bt_col[uu];
-            }
-#pragma unroll
-            for (int w = 0; w < 4; ++w) vq[w] = V[sq[w]];
-#pragma unroll
-            for (int w = 0; w < 4; ++w)
-                if (u + w < u1) acc += vq[w] * Yl[(size_t)c * ne + cq[w]];
-        }
-        Sm[(size_t)c * me + k] = acc;
+        Sm[(size_t)c * me + k] = cond_row_dot(S, V, l0 + k, Yl + (size_t)c * ne);
     }
+    if (sizeof(TT) == 4 && S.cond_fac != nullptr) {  // kept for the refinement's solves
+        float* fac = S.cond_fac + S.cond_fac_off[ce];
+        for (int q = t; q < ne * ne; q += blockDim.x) {
+            const int i = q / ne, j = q - ne * (q / ne);
+            fac[q] = (float)M[i * lda + j];
+        }
+        for (int i = t; i < ne; i += blockDim.x) S.cond_fac_row[r0 + i] = ph[i];
+    }
+}
+
+// A refinement sweep's element solve with the factors of this iteration's k_cond_factor_f32: the
+// matrix has not changed, so Y_B and the S_e block stand and only the right-hand side's column is
+// new.  y = K_e^-1 r_e by the FP64-accumulating triangular solves of the fused form's refinement,
+// one workgroup per element, bound by their serial chain over 16-row blocks.  Refactoring in every
+// sweep took 124 us of each.
+__host__ __device__ inline int cond_resolve_bytes(int ne) {
+    return align16(ne * (ne | 1) * 4) + align16(ne * 4) + 2 * align16(ne * 8);
+}
+__global__ void __launch_bounds__(kThreads) k_cond_resolve_f32(DevSys S, const double* rin) {
+    extern __shared__ __align__(16) char sm[];
+    const int ce = blockIdx.x, t = threadIdx.x;
+    const int b = S.cond_elem_block[ce];
+    if (!S.model_active[S.block_model[b]]) return;
+    const double* V = S.crs_val + S.crs_nz_off[b];
+    const int r0 = S.cond_rows_off[ce], ne = S.cond_rows_off[ce + 1] - r0;
+    const int l0 = S.cond_lam_off[ce], me = S.cond_lam_off[ce + 1] - l0;
+    const int lda = ne | 1;
+    float* M = reinterpret_cast<float*>(sm);
+    int off = align16(ne * lda * 4);
+    int* ph = reinterpret_cast<int*>(sm + off);
+    off += align16(ne * 4);
+    double* r = reinterpret_cast<double*>(sm + off);
+    off += align16(ne * 8);
+    double* y = reinterpret_cast<double*>(sm + off);
+    const float* fac = S.cond_fac + S.cond_fac_off[ce];
+    for (int q0 = t; q0 < ne * ne; q0 += 8 * blockDim.x) {  // eight loads in flight per thread
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = fac[q0 + u * (int)blockDim.x < ne * ne ? q0 + u * (int)blockDim.x : q0];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int q = q0 + u * (int)blockDim.x;
+            if (q < ne * ne) M[(q / ne) * lda + q % ne] = v[u];
+        }
+    }
+    for (int i = t; i < ne; i += blockDim.x) {
+        ph[i] = S.cond_fac_row[r0 + i];
+        r[i] = rin[S.block_vec_off[b] + S.cond_rows[r0 + i]];
+    }
+    __syncthreads();
+    lu_solve<float>(M, ne, lda, ph, r, y);
+    double* Y = S.Ybuf + S.cond_Y_off[ce] + (size_t)me * ne;
+    for (int i = t; i < ne; i += blockDim.x) Y[i] = y[i];
+    double* Sm = S.Sbuf + S.cond_S_off[ce] + (size_t)me * me;
+    for (int k = t; k < me; k += blockDim.x) Sm[k] = cond_row_dot(S, V, l0 + k, y);
 }
 __global__ void __launch_bounds__(kThreads) k_cond_factor_f64(DevSys S, const double* rin) {
     cond_factor_body<double>(S, rin);
@@ -3460,6 +3521,8 @@ hipError_t set_lds_limits(size_t bytes) {
     if (e != hipSuccess) return e;
     e = hipFuncSetAttribute((const void*)k_cond_factor_f32, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
     if (e != hipSuccess) return e;
+    e = hipFuncSetAttribute((const void*)k_cond_resolve_f32, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+    if (e != hipSuccess) return e;
     return hipFuncSetAttribute((const void*)k_plain_solve, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
 }
 
@@ -3548,6 +3611,10 @@ void launch_cond_factor(const DevSys& S, size_t lds, bool fp32, const double* ri
         hipLaunchKernelGGL(k_cond_factor_f32, dim3(S.num_cond_elems), dim3(kThreads), lds, st, S, rin);
     else
         hipLaunchKernelGGL(k_cond_factor_f64, dim3(S.num_cond_elems), dim3(kThreads), lds, st, S, rin);
+}
+size_t cond_resolve_lds(int ne) { return (size_t)cond_resolve_bytes(ne); }
+void launch_cond_resolve(const DevSys& S, size_t lds, const double* rin, hipStream_t st) {
+    hipLaunchKernelGGL(k_cond_resolve_f32, dim3(S.num_cond_elems), dim3(kThreads), lds, st, S, rin);
 }
 void launch_cond_interface(const DevSys& S, int b, int nz, const int* colour_sizes, int ncolour, const double* rin,
                            hipStream_t st) {

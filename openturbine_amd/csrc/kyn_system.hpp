@@ -178,6 +178,11 @@ struct DevSys {
     const int64_t* cond_Y_off;        // into Ybuf: n_e x (m_e + 1), column-major (K_e^-1 [B_e^T | b_e])
     const int64_t* cond_S_off;        // into Sbuf: m_e x (m_e + 1), column-major (B_e K_e^-1 [B_e^T | b_e])
     double *Ybuf, *Sbuf;
+    // FP32 option with refinement (else null): the elements' FP32 factors, [n_e][n_e] by physical
+    // row, and their row maps (at cond_rows_off), from the iteration's factorization for its sweeps
+    float* cond_fac;
+    const int64_t* cond_fac_off;
+    int* cond_fac_row;
     const int* block_z_off;           // [b+1] into cond_z (interface rows of the block, ascending)
     const int* cond_z;
     const int* block_ce_begin;        // [b+1] condensed elements of the block
