@@ -1293,6 +1293,7 @@ kyn_system kyn_system_create(const kyn_model* models, size_t num_models, const k
                     work.insert(work.end(), {m, -1});
                 }
             }
+            S.elem_split = 3 * S.num_elems <= cus;
             S.fused_work = Ar.up(work);
             S.num_fused_work = static_cast<int>(work.size() / 2);
             S.fused_ticket = split ? Ar.zeros<int>(1) : nullptr;

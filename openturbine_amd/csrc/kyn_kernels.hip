@@ -369,28 +369,28 @@ __device__ __forceinline__ void contract_mfma_f32(const DevSys& S, char* sm, con
 // Node-pair contraction on the VALU (the FP64 tangent's, and the FP32 tangent's where the tuning
 // table picks it for the element size).
 // ---------------------------------------------------------------------------------------
-template <typename TT, bool kFused>
+template <typename TT, bool kFused, int NB = 3>
 __device__ __forceinline__ void contract_valu(const DevSys& S, char* sm, const Lay& L, int n, int N, int Q,
-                                              const int* loc, double* mat_out) {
+                                              const int* loc, double* mat_out, int j0 = 0) {
     const int tid = threadIdx.x;
     const TT* qpM = reinterpret_cast<const TT*>(sm + L.qpM);
     const TT* phiT = reinterpret_cast<const TT*>(sm + L.phiT);
     const double* tr = reinterpret_cast<const double*>(sm + L.tr);
     // ---- contraction, one pass over the QPs, no barrier
-    // Thread t < 252 owns component cc = t % 36 = (r, s) and nodes j = t / 36 + 7 b (b < 3);
+    // Thread t < 252 owns component cc = t % 36 = (r, s) and nodes j = j0 + t / 36 + 7 b (b < NB);
     // per QP it forms its own R0_q[j][cc], R1_q[j][cc] from row r of the QP matrices and
     // column s of T_j, then accumulates S_ij[cc] += phi_i R0 + phi'_i R1 for every row i
     // (the QP's phi pairs: broadcast vector loads, all rows at once).  Each R entry is formed by
     // exactly one thread.
-    const int cc = tid % 36, jg = tid / 36;
+    const int cc = tid % 36, jg = j0 + tid / 36;
     const bool active = tid < kContractThreads;
     const int r_ = cc / 6, s_ = cc - 6 * (cc / 6);
     const bool rot = s_ >= 3;
     const int col0 = rot ? 3 : 0;  // columns of A/P/O/C combined with T_j's column (s - 3)
-    TT tc[3][3];
-    int jc[3];
+    TT tc[NB][3];
+    int jc[NB];
 #pragma unroll
-    for (int b = 0; b < 3; ++b) {
+    for (int b = 0; b < NB; ++b) {
         const int j = jg + 7 * b;
         const bool ok = active && j < N;
         jc[b] = ok ? j : 0;
@@ -398,11 +398,11 @@ __device__ __forceinline__ void contract_valu(const DevSys& S, char* sm, const L
         for (int u = 0; u < 3; ++u)
             tc[b][u] = !ok ? TT(0) : (rot ? (TT)tr[j * 9 + u * 3 + (s_ - 3)] : (u == s_ ? TT(1) : TT(0)));
     }
-    TT acc[kMaxElemNodes][3];
+    TT acc[kMaxElemNodes][NB];
 #pragma unroll
     for (int i = 0; i < kMaxElemNodes; ++i)
 #pragma unroll
-        for (int b = 0; b < 3; ++b) acc[i][b] = TT(0);
+        for (int b = 0; b < NB; ++b) acc[i][b] = TT(0);
     const int Nu = __builtin_amdgcn_readfirstlane(N);  // uniform: a scalar branch per row group
     for (int q = 0; q < Q; ++q) {
         const TT* M6 = qpM + (size_t)q * 6 * 36 + r_ * 6;
@@ -416,9 +416,9 @@ __device__ __forceinline__ void contract_valu(const DevSys& S, char* sm, const L
         }
         const TT rm = M6[72 + s_];
         const TT* ph = phiT + (size_t)q * kPhiStride;
-        TT pj[3], dj[3];
+        TT pj[NB], dj[NB];
 #pragma unroll
-        for (int b = 0; b < 3; ++b) {
+        for (int b = 0; b < NB; ++b) {
             pj[b] = ph[jc[b] * 2];
             dj[b] = ph[jc[b] * 2 + 1];
         }
@@ -432,9 +432,9 @@ __device__ __forceinline__ void contract_valu(const DevSys& S, char* sm, const L
 #pragma unroll
             for (int e = 0; e < VW; ++e) phv[c * VW + e] = v[e];
         }
-        TT R0[3], R1[3];
+        TT R0[NB], R1[NB];
 #pragma unroll
-        for (int b = 0; b < 3; ++b) {
+        for (int b = 0; b < NB; ++b) {
             TT v0 = pj[b] * rm, v1 = TT(0);
 #pragma unroll
             for (int u = 0; u < 3; ++u) {
@@ -452,7 +452,7 @@ __device__ __forceinline__ void contract_valu(const DevSys& S, char* sm, const L
                 for (int i = i0; i < i0 + 3 && i < kMaxElemNodes; ++i) {
                     const TT pi = phv[i * 2], di = phv[i * 2 + 1];
 #pragma unroll
-                    for (int b = 0; b < 3; ++b) acc[i][b] += pi * R0[b] + di * R1[b];
+                    for (int b = 0; b < NB; ++b) acc[i][b] += pi * R0[b] + di * R1[b];
                 }
             }
         }
@@ -477,7 +477,7 @@ __device__ __forceinline__ void contract_valu(const DevSys& S, char* sm, const L
                 if (i < N) {
                     const int row = loc[i] + r_;
 #pragma unroll
-                    for (int b = 0; b < 3; ++b) {
+                    for (int b = 0; b < NB; ++b) {
                         const int j = jg + 7 * b;
                         if (j < N) A[row * L.lda + loc[j] + s_] = acc[i][b] * cond;
                     }
@@ -492,7 +492,7 @@ __device__ __forceinline__ void contract_valu(const DevSys& S, char* sm, const L
             for (int i = 0; i < kMaxElemNodes; ++i) {
                 if (i < N) {
 #pragma unroll
-                    for (int b = 0; b < 3; ++b) {
+                    for (int b = 0; b < NB; ++b) {
                         const int j = jg + 7 * b;
                         if (j < N) out[(size_t)(i * N + j) * 36 + cc] = (double)acc[i][b];
                     }
@@ -512,10 +512,12 @@ __device__ __forceinline__ void contract_valu(const DevSys& S, char* sm, const L
 // ---------------------------------------------------------------------------------------
 //   model: the element's model where the caller knows it (one load for the gravity vector
 //           instead of the element -> node -> block -> model chain), else -1.
-template <typename TT, bool kFused, bool kOwnTangent = kFused>
+//   kSplit: this workgroup forms the columns of nodes 7 part .. 7 part + 6 only (FP64 VALU
+//           contraction), part 0 the residual too.
+template <typename TT, bool kFused, bool kOwnTangent = kFused, bool kSplit = false>
 __device__ __forceinline__ void element_phase(const DevSys& S, int e, char* sm, const Lay& L, int n,
                                               double* res_out = nullptr, double* mat_out = nullptr,
-                                              int model = -1) {
+                                              int model = -1, int part = 0) {
     const int tid = threadIdx.x;
     const int N = S.elem_N[e], Q = S.elem_Q[e];
     const int noff = S.elem_node_off[e];
@@ -596,6 +598,7 @@ __device__ __forceinline__ void element_phase(const DevSys& S, int e, char* sm, 
             // interpolate_to_quadrature_point_for_inertia.hpp:19-40
             double r[4] = {0., 0., 0., 0.}, ud[3] = {0., 0., 0.}, om[3] = {0., 0., 0.},
                    omd[3] = {0., 0., 0.};
+#pragma unroll 3
             for (int k = 0; k < N; ++k) {
                 const double p = phi[k * Q + q];
 #pragma unroll
@@ -613,6 +616,7 @@ __device__ __forceinline__ void element_phase(const DevSys& S, int e, char* sm, 
         } else {
             // interpolate_to_quadrature_point_for_stiffness.hpp:19-41
             double r[4] = {0., 0., 0., 0.}, rp[4] = {0., 0., 0., 0.}, up[3] = {0., 0., 0.};
+#pragma unroll 3
             for (int k = 0; k < N; ++k) {
                 const double p = phi[k * Q + q];
                 const double dp = dphi[k * Q + q] / J;
@@ -634,12 +638,13 @@ __device__ __forceinline__ void element_phase(const DevSys& S, int e, char* sm, 
     KYN_PHASE_MARK(2);
 
     // ---- residual (integrate_residual_vector.hpp:32-50)
-    for (int t = tid; t < 6 * N; t += blockDim.x) {
+    for (int t = kSplit && part > 0 ? 6 * N : tid; t < 6 * N; t += blockDim.x) {
         const int k = t / 6, c = t - 6 * (t / 6);
         // HBM operands first: their latency runs under the QP loop
         const double fx = S.node_FX[(size_t)(noff + k) * 6 + c];
         const double fk = kFused ? S.f[S.elem_nodes[noff + k] * 6 + c] : 0.;
         double acc = 0.;
+#pragma unroll 4  // four points' LDS loads in flight (the sum's order is the loop's)
         for (int q = 0; q < Q; ++q) {
             const double w = wq[q];
             const double cc = w * dphi[k * Q + q];
@@ -666,6 +671,8 @@ __device__ __forceinline__ void element_phase(const DevSys& S, int e, char* sm, 
                 contract_mfma_f32<kFused, false>(S, sm, L, n, N, Q, loc, mat_out);
         } else
             contract_valu<TT, kFused>(S, sm, L, n, N, Q, loc, mat_out);
+    } else if constexpr (kSplit) {
+        contract_valu<TT, kFused, 1>(S, sm, L, n, N, Q, loc, mat_out, 7 * part);
     } else {
         contract_valu<TT, kFused>(S, sm, L, n, N, Q, loc, mat_out);
     }
@@ -764,8 +771,8 @@ __device__ __forceinline__ bool is_zero(double v) { return (__double_as_longlong
 // A single wave issues about one instruction per four cycles, so a column costs its instruction
 // count: the search is one integer reduction over the magnitudes' high words, masks are bitwise
 // selects on done, and the logical rows are touched only by an interchange.  Panels per block of
-// the mixed FP64 ensemble (n = 42 .. 132): 61k cycles, 79k with reductions of doubles and of row
-// keys; the whole LU 139k -> 105k.
+// the mixed FP64 ensemble (n = 42 .. 132): 67k cycles, 79k with reductions of doubles and of row
+// keys; the whole LU 139k -> 113k.
 template <typename TT, int NS, bool kFull, int J>
 __device__ __forceinline__ void panel_columns(TT (&P)[NS][kPanel], int (&lg)[NS], int (&done)[NS], int (&pl)[kPanel],
                                               int c0, int w, int lane) {
@@ -1002,9 +1009,9 @@ __device__ __forceinline__ void u_rows_group_fma(const float* Lc, float (&u)[kPa
 
 // 16 x 16 x 4 matrix-core products: A operand row lane % 16, k = lane / 16, B operand column
 // lane % 16, same k.  Both types accumulate c + a_0 b_0 + ... + a_3 b_3 like a chain of FMAs in
-// ascending k (the same bits on 5e6 random entries with exponents within 2^40 of each other), the
-// update loop's sequence; on the mixed FP64 ensemble 7 of 192 blades' first increments end in
-// other last bits than with the loop, at the same distance from a 64-bit solve.
+// ascending k (the same bits on 5e6 random entries), so a trailing update on the matrix cores is
+// the update loop's FMA sequence; the mixed ensembles' states keep every bit (FP64 256 rotors, FP32
+// 1024, 6 steps).
 template <typename TT>
 struct MfmaTile;
 template <>
@@ -1129,7 +1136,7 @@ __device__ __forceinline__ void lu_lookahead(TT* A, int n, int lda, int c0, int 
 // mapping is this panel's: the next panel's factorization (wave 0, possibly running meanwhile)
 // permutes rows among logical c0 + w .. n - 1 only and writes the other buffer.
 // Runs within one wave: its LDS writes are seen by its own later reads without a barrier.
-// Look-ahead and trailing update per block of the mixed FP64 ensemble: 69k cycles, 83k on the VALU
+// Look-ahead and trailing update per block of the mixed FP64 ensemble: 70k cycles, 83k on the VALU
 // (a row per lane, two columns at a time, u broadcast from LDS).
 template <typename TT>
 __device__ __forceinline__ void lu_apply(TT* A, int n, int lda, int c0, int w, int ja, int jb, int g, int gs,
@@ -2497,6 +2504,21 @@ __global__ void __launch_bounds__(kThreads) k_plain_element(DevSys S, int Nm, in
                                  S.elem_mat + S.elem_mat_off[e]);
 }
 
+// The same with three workgroups per element, each forming the columns of seven nodes (a register
+// tile of 21 x 1 per thread instead of 21 x 3): the gather, QP values and operand loads are
+// repeated, the FMAs and stores divided.  For systems whose elements leave most CUs idle (one
+// workgroup's LDS fills a CU): used while three workgroups per element fit the chip at once.
+// One element's terms through the host call (21 nodes, 40 points): 80.8 -> 68.9 us.
+__global__ void __launch_bounds__(kThreads) k_plain_element_split(DevSys S, int Nm, int Qm) {
+    extern __shared__ __align__(16) char sm[];
+    const Lay L = make_layout(Nm, Qm, 1, 0, false, 8, false);
+    const int e = blockIdx.x, part = blockIdx.y;
+    const int m = S.block_model[S.node_block[S.elem_nodes[S.elem_node_off[e]]]];
+    if (!S.model_active[m] || 7 * part >= S.elem_N[e]) return;
+    element_phase<double, false, false, true>(S, e, sm, L, 0, S.elem_res + (size_t)S.elem_node_off[e] * 6,
+                                              S.elem_mat + S.elem_mat_off[e], m, part);
+}
+
 // FP32-tangent option of the plain form: QP matrices in FP32 and the node-pair contraction on
 // the matrix cores (as in the fused FP32 form), element terms stored in FP64.
 __global__ void __launch_bounds__(kThreads) k_plain_element_f32(DevSys S, int Nm, int Qm) {
@@ -2510,11 +2532,13 @@ __global__ void __launch_bounds__(kThreads) k_plain_element_f32(DevSys S, int Nm
 }
 
 // One element's residual and iteration matrix at the current state, with its own tangent
-// blocks (the no-allocation element-terms entry point): res [N][6], mat [N][N][36].
+// blocks (the no-allocation element-terms entry point): res [N][6], mat [N][N][36].  Three
+// workgroups, as k_plain_element_split.
 __global__ void __launch_bounds__(kThreads) k_element_terms(DevSys S, int Nm, int Qm, int e, double* res, double* mat) {
     extern __shared__ __align__(16) char sm[];
     const Lay L = make_layout(Nm, Qm, 1, 0, false, 8, false);
-    element_phase<double, false, true>(S, e, sm, L, 0, res, mat);
+    if (7 * (int)blockIdx.x >= S.elem_N[e]) return;
+    element_phase<double, false, true, true>(S, e, sm, L, 0, res, mat, -1, blockIdx.x);
 }
 
 // UpdateSystemVariablesMasses / UpdateSystemVariablesSprings
@@ -3511,6 +3535,8 @@ hipError_t set_lds_limits(size_t bytes) {
     if (e != hipSuccess) return e;
     e = hipFuncSetAttribute((const void*)k_plain_element, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
     if (e != hipSuccess) return e;
+    e = hipFuncSetAttribute((const void*)k_plain_element_split, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+    if (e != hipSuccess) return e;
     e = hipFuncSetAttribute((const void*)k_element_terms, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
     if (e != hipSuccess) return e;
     e = hipFuncSetAttribute((const void*)k_plain_element_f32, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
@@ -3564,7 +3590,7 @@ hipError_t element_terms_scratch(int device, double** ptr) {
 }
 
 void launch_element_terms(const DevSys& S, int Nm, int Qm, int e, double* res, double* mat, hipStream_t st) {
-    hipLaunchKernelGGL(k_element_terms, dim3(1), dim3(kThreads), element_lds_bytes(Nm, Qm), st, S, Nm, Qm, e, res, mat);
+    hipLaunchKernelGGL(k_element_terms, dim3(3), dim3(kThreads), element_lds_bytes(Nm, Qm), st, S, Nm, Qm, e, res, mat);
 }
 
 void launch_advance_slot(const DevSys& S, hipStream_t st) {
@@ -3583,6 +3609,9 @@ void launch_plain_iteration(const DevSys& S, int Nm, int Qm, int nm, int iter, b
         if (S.precision)
             hipLaunchKernelGGL(k_plain_element_f32, dim3(S.num_elems), dim3(kThreads),
                                (size_t)make_layout(Nm, Qm, 1, 0, false, 4, false).total, st, S, Nm, Qm);
+        else if (S.elem_split)
+            hipLaunchKernelGGL(k_plain_element_split, dim3(S.num_elems, 3), dim3(kThreads), element_lds_bytes(Nm, Qm), st,
+                               S, Nm, Qm);
         else
             hipLaunchKernelGGL(k_plain_element, dim3(S.num_elems), dim3(kThreads), element_lds_bytes(Nm, Qm), st, S, Nm,
                                Qm);

@@ -116,6 +116,7 @@ struct DevSys {
     double* node_FX;                           // [sum N][6]
     double* elem_res;                          // [sum N][6]
     double* elem_mat;                          // [sum N^2][36] (plain form)
+    int elem_split;  // plain form, FP64: three workgroups per element (they all fit the chip at once)
 
     // ---- point masses (src/elements/masses/masses.hpp) and springs (src/elements/springs/springs.hpp)
     int num_masses, num_springs;
