@@ -266,7 +266,10 @@ struct kyn_system_s {
     double *rfull{}, *dfull{};  // refinement of condensed blocks: residual and correction (rhs layout)
     double* motion{};           // packed x, q, v, vd for kyn_get_motion (allocated on first use)
     float* r32{};
-    std::vector<int> model_active_host;
+    const int* model_active_host{};  // large blocks: the models still iterating (in host_flags)
+    // pinned host copies of what a step reports, written in the step's stream before its one wait:
+    // device error flags, any_active, then per model the status and (large blocks) whether it iterates
+    int* host_flags{};
     // graph of one fused step
     hipGraph_t graph{};
     hipGraphExec_t graph_exec{};
@@ -281,6 +284,7 @@ struct kyn_system_s {
         if (ek1) (void)hipEventDestroy(ek1);
         if (blas) (void)rocblas_destroy_handle(blas);
         if (stream) (void)hipStreamDestroy(stream);
+        if (host_flags) (void)hipHostFree(host_flags);
     }
 };
 
@@ -970,11 +974,19 @@ void solve_large_blocks(kyn_system_s* s) {
     }
 }
 
+// The step's report to pinned memory, behind the step in its stream: a blocking copy per item after
+// the step cost ~15 us each, a third of the host's share of a small step.
+void read_back(kyn_system_s* s, const int* per_model) {
+    hip_check(hipMemcpyAsync(s->host_flags, s->S.dev_error, sizeof(int), hipMemcpyDeviceToHost, s->stream), "D2H");
+    hip_check(hipMemcpyAsync(s->host_flags + 2, per_model, s->num_models * sizeof(int), hipMemcpyDeviceToHost, s->stream),
+              "D2H");
+}
+
 // Device error flags raised by a kernel that gave up a bounded wait: reported (and cleared)
 // after the step, as an error of the step.
+// Called after the wait that ended the step (read_back is the copy that precedes it).
 void check_device_errors(kyn_system_s* s) {
-    int flags = 0;
-    hip_check(hipMemcpy(&flags, s->S.dev_error, sizeof(int), hipMemcpyDeviceToHost), "D2H");
+    const int flags = s->host_flags[0];
     if (flags == 0) return;
     const int zero = 0;
     hip_check(hipMemcpy(s->S.dev_error, &zero, sizeof(int), hipMemcpyHostToDevice), "H2D");
@@ -1000,7 +1012,9 @@ int run_step(kyn_system_s* s, bool solve = true) {
         hip_check(hipGetLastError(), "k_plain_predict launch");
         int count = 0;
         const bool large = !s->large_blocks.empty();
-        if (large) s->model_active_host.assign(s->num_models, 1);
+        int* active = s->host_flags + 2 + s->num_models;
+        s->model_active_host = active;
+        if (large) std::fill(active, active + s->num_models, 1);
         for (int iter = 0; iter < S.p.max_iter; ++iter) {
             kyn::launch_plain_iteration(S, s->Nm, s->Qm, s->nm, iter, solve, s->stream, s->ek0, s->ek1, large);
             hip_check(hipGetLastError(), "plain iteration launch");
@@ -1009,18 +1023,16 @@ int run_step(kyn_system_s* s, bool solve = true) {
                 solve_large_blocks(s);
                 kyn::launch_plain_update(S, iter, s->stream);
                 hip_check(hipGetLastError(), "k_plain_update launch");
-                hip_check(hipMemcpyAsync(s->model_active_host.data(), S.model_active, s->num_models * sizeof(int),
-                                         hipMemcpyDeviceToHost, s->stream),
+                hip_check(hipMemcpyAsync(active, S.model_active, s->num_models * sizeof(int), hipMemcpyDeviceToHost, s->stream),
                           "D2H");
             }
-            int any = 0;
-            hip_check(hipMemcpyAsync(&any, S.any_active, sizeof(int), hipMemcpyDeviceToHost, s->stream), "D2H");
+            hip_check(hipMemcpyAsync(s->host_flags + 1, S.any_active, sizeof(int), hipMemcpyDeviceToHost, s->stream), "D2H");
             hip_check(hipStreamSynchronize(s->stream), "sync");
             float ms = 0.f;
             hip_check(hipEventElapsedTime(&ms, s->ek0, s->ek1), "elapsed");
             kms += ms;
             ++count;
-            if (!any) break;
+            if (!s->host_flags[1]) break;
         }
         if (solve) {
             kyn::launch_plain_epilogue(S, s->stream);
@@ -1029,6 +1041,7 @@ int run_step(kyn_system_s* s, bool solve = true) {
         if (count > 0) kms /= static_cast<float>(count);
     }
     hip_check(hipEventRecord(s->ev1, s->stream), "event");
+    read_back(s, S.model_status);
     hip_check(hipStreamSynchronize(s->stream), "sync");
     float ms = 0.f;
     hip_check(hipEventElapsedTime(&ms, s->ev0, s->ev1), "elapsed");
@@ -1039,10 +1052,8 @@ int run_step(kyn_system_s* s, bool solve = true) {
     s->last_kernel_ms = kms;
     check_device_errors(s);
     if (!solve) return KYN_OK;
-    std::vector<int> st(s->num_models);
-    hip_check(hipMemcpy(st.data(), S.model_status, st.size() * sizeof(int), hipMemcpyDeviceToHost), "D2H");
-    for (int v : st)
-        if (v != 0) return KYN_NOT_CONVERGED;
+    for (size_t m = 0; m < s->num_models; ++m)
+        if (s->host_flags[2 + m] != 0) return KYN_NOT_CONVERGED;
     return KYN_OK;
 }
 
@@ -1769,6 +1780,9 @@ kyn_system kyn_system_create(const kyn_model* models, size_t num_models, const k
         sys->con_block = B.con_block;
         sys->model_gdof_to_block_vec = B.gdof_maps;
 
+        hip_check(hipHostMalloc(reinterpret_cast<void**>(&sys->host_flags), (2 + 2 * num_models) * sizeof(int),
+                                hipHostMallocDefault),
+                  "hipHostMalloc");
         hip_check(hipStreamCreateWithFlags(&sys->stream, hipStreamNonBlocking), "hipStreamCreate");
         if (sys->blas && rocblas_set_stream(sys->blas, sys->stream) != rocblas_status_success)
             throw KynError(KYN_ERR_HIP, "rocblas_set_stream failed");
@@ -1863,6 +1877,7 @@ int kyn_step_many(kyn_system s, size_t num_steps, int use_graph) {
             }
         }
         hip_check(hipEventRecord(s->ev1, s->stream), "event");
+        read_back(s, S.model_fail_total);
         hip_check(hipStreamSynchronize(s->stream), "sync");
         float total = 0.f, kern = 0.f;
         hip_check(hipEventElapsedTime(&total, s->ev0, s->ev1), "elapsed");
@@ -1875,10 +1890,8 @@ int kyn_step_many(kyn_system s, size_t num_steps, int use_graph) {
         s->last_step_ms = total;
         s->last_kernel_ms = kern / static_cast<float>(num_steps);
         check_device_errors(s);
-        std::vector<int> fails(s->num_models);
-        hip_check(hipMemcpy(fails.data(), S.model_fail_total, fails.size() * sizeof(int), hipMemcpyDeviceToHost), "D2H");
-        for (int f : fails)
-            if (f != 0) return KYN_NOT_CONVERGED;
+        for (size_t m = 0; m < s->num_models; ++m)
+            if (s->host_flags[2 + m] != 0) return KYN_NOT_CONVERGED;
         return KYN_OK;
     });
 }
@@ -1932,11 +1945,15 @@ int kyn_set_constraint_displacement(kyn_system s, size_t id, const double disp[7
 int kyn_set_constraint_displacements(kyn_system s, size_t count, const size_t* ids, const double* disp) {
     return guarded([&] {
         if (!s || !ids || !disp) throw KynError(KYN_ERR_INVALID, "null argument");
-        for (size_t k = 0; k < count; ++k) {
-            if (ids[k] >= s->num_cons) throw KynError(KYN_ERR_INVALID, "constraint id out of range");
-            hip_check(hipMemcpyAsync(s->S.con_input + ids[k] * 7, disp + 7 * k, 7 * sizeof(double),
+        for (size_t k = 0; k < count;) {  // a copy per run of consecutive ids
+            size_t run = 0;
+            for (; k + run < count && ids[k + run] == ids[k] + run; ++run)
+                if (ids[k + run] >= s->num_cons) break;
+            if (run == 0) throw KynError(KYN_ERR_INVALID, "constraint id out of range");
+            hip_check(hipMemcpyAsync(s->S.con_input + ids[k] * 7, disp + 7 * k, run * 7 * sizeof(double),
                                      hipMemcpyHostToDevice, s->stream),
                       "H2D");
+            k += run;
         }
         hip_check(hipStreamSynchronize(s->stream), "sync");
         return KYN_OK;
