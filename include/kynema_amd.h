@@ -214,6 +214,13 @@ int kyn_debug_set_wait_limit(kyn_system s, int polls);
  * tuning table (openturbine_amd/autotune.py); this call overrides it (the autotuner, tests).
  * No counterpart in the reference. */
 int kyn_debug_set_contraction_mask(kyn_system s, unsigned mask);
+/* Workgroups of the fused step's launch (one per model, or one per block where models are split) and
+ * per element of the plain form's element kernel.  No counterpart in the reference. */
+int kyn_debug_get_launch(kyn_system s, int* fused_workgroups, int* element_workgroups);
+/* Launches the fused step with the workgroups of at most `per_model` blocks of every model (its last
+ * ones): what a split step does when the others find no room on the GPU (tests).  No counterpart in
+ * the reference. */
+int kyn_debug_set_fused_workgroups(kyn_system s, int per_model);
 int kyn_get_element_terms(kyn_system s, size_t element, double* residual /* [N][6] */,
                           double* system_matrix /* [N][N][36] */);
 /* The CRS matrix of a model whose dofs form one large block (plain form), in the reference's

@@ -11,6 +11,7 @@
 
 #include <algorithm>
 #include <array>
+#include <climits>
 #include <cmath>
 #include <cstring>
 #include <functional>
@@ -249,6 +250,7 @@ struct kyn_system_s {
     std::vector<int> node_block, node_local;
     std::vector<int> con_local, con_rows, con_model_row, con_block;
     std::vector<std::vector<int>> model_gdof_to_block_vec;  // per model: global dof -> rhs index
+    std::vector<int> fused_work;  // the fused launch's list
     double* saved{};  // saved state (CopyStateData), on the device; allocated on first use
     bool has_saved{false};
     // large blocks (library LU): block ids, sizes, matrix offsets, pivots, scratch vectors
@@ -852,9 +854,14 @@ double* field_ptr(kyn_system_s* s, int field, int& width) {
 // Whether a fused launch of num_models models gives every block a workgroup of its own: while the
 // models are no more than the workgroups the chip holds (one per CU in FP64, two in FP32).  Beyond
 // that the models fill it by themselves, and a block that waits for a larger one of its model holds
-// a place another model could use.  Measured, 3-blade rotors of mixed blade sizes, us per step
-// unsplit / split: FP64 96 rotors 2940 / 1442, 256 2963 / 2725, 300 3132 / 3275, 512 4247 / 5239;
-// FP32 96 2303 / 942, 256 2330 / 1498, 512 2442 / 2328, 700 2914 / 3142, 1536 5028 / 6526.
+// a place another model could use.  Measured, us per step unsplit / split, 3-blade rotors of mixed
+// blade sizes (N = 6 .. 21): FP64 96 rotors 2940 / 1442, 256 2963 / 2725, 300 3132 / 3275, 512 4247 /
+// 5239; FP32 96 2303 / 942, 256 2330 / 1498, 512 2442 / 2328, 700 2914 / 3142, 1536 5028 / 6526.  Rotors
+// of equal blades have no larger block to wait for and still gain a little beyond the line (N = 11 /
+// 21: FP64 512 3581 / 3399 and 6500 / 6239, 1024 6682 / 6387 and 12568 / 11868; FP32 1024 3024 / 2844
+// and 6239 / 5736), which the rule gives up.  It looks at one system: several stepping at once from
+// threads each split by their own size (two of 256 FP64 rotors 3.80 ms unsplit, 4.10 ms split for a
+// step of both; four of 96 6.06 / 3.56; two of 256 in FP32 2.46 / 1.91).
 bool fused_split_models(size_t num_models, int cus, bool fp32) {
     return num_models <= static_cast<size_t>(cus) * (fp32 ? 2 : 1);
 }
@@ -1288,26 +1295,30 @@ kyn_system kyn_system_create(const kyn_model* models, size_t num_models, const k
             std::vector<int> order(num_models);
             for (size_t m = 0; m < num_models; ++m) order[m] = static_cast<int>(m);
             std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return cost[x] > cost[y]; });
-            // One workgroup per block where the models do not fill the chip by themselves (see
-            // fused_split_models for the line); every block of a split model must be able to run at once
             int cus = 0;
             hip_check(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev), "attr");
-            const bool split_all = sys->exec_mode == KYN_EXEC_FUSED && fused_split_models(num_models, cus, S.precision != 0);
-            std::vector<int> work;
-            bool split = false;
+            int least_blocks = INT_MAX, most_blocks = 0;
+            for (size_t m = 0; m < num_models; ++m) {
+                least_blocks = std::min(least_blocks, B.model_block_end[m] - B.model_block_begin[m]);
+                most_blocks = std::max(most_blocks, B.model_block_end[m] - B.model_block_begin[m]);
+            }
+            const bool split = sys->exec_mode == KYN_EXEC_FUSED && fused_split_models(num_models, cus, S.precision != 0) &&
+                               least_blocks >= 1 && most_blocks >= 2 && most_blocks <= kyn::kMaxSplitBlocks;
             for (int m : order) {
-                const int nb = B.model_block_end[m] - B.model_block_begin[m];
-                if (split_all && nb > 1 && nb <= std::min(kyn::kMaxSplitBlocks, cus)) {
-                    split = true;
-                    for (int k = 0; k < nb; ++k) work.insert(work.end(), {m, k});
-                } else {
-                    work.insert(work.end(), {m, -1});
-                }
+                const int nb = split ? B.model_block_end[m] - B.model_block_begin[m] : 1;
+                for (int k = 0; k < nb; ++k) sys->fused_work.insert(sys->fused_work.end(), {m, k});
             }
             S.elem_split = 3 * S.num_elems <= cus;
-            S.fused_work = Ar.up(work);
-            S.num_fused_work = static_cast<int>(work.size() / 2);
-            S.fused_ticket = split ? Ar.zeros<int>(1) : nullptr;
+            S.fused_work = Ar.up(sys->fused_work);
+            S.num_fused_work = static_cast<int>(sys->fused_work.size() / 2);
+            // More workgroups than the chip holds at once: entries by ticket, in the order workgroups
+            // start, so that the next one goes to whichever XCD has room first (workgroup i is tied to
+            // XCD i % 8; 96 FP64 rotors 1.31 -> 1.20 ms a step, 256 2.31 -> 2.27).  With places for all
+            // the block index is as good an order and the atomic's latency is saved (96 FP32 rotors,
+            // refined in every iteration, 1.08 -> 0.99 ms).
+            const size_t places = static_cast<size_t>(cus) * (S.precision != 0 ? 2 : 1);
+            S.fused_ticket = split && static_cast<size_t>(S.num_fused_work) > places ? Ar.zeros<int>(1) : nullptr;
+            S.fused_claim = split ? Ar.zeros<int>(B.block_n.size()) : nullptr;
             S.fused_xch = split ? Ar.up(std::vector<unsigned long long>(B.block_n.size() * static_cast<size_t>(S.p.max_iter),
                                                                        kyn::kXchEmpty))
                                 : nullptr;
@@ -2198,6 +2209,30 @@ int kyn_read_restart(kyn_system s, size_t model, const unsigned char* in, size_t
             hip_check(hipMemcpy(p + n0 * w, in + off, n * w * sizeof(double), hipMemcpyHostToDevice), "H2D");
             off += n * w * sizeof(double);
         }
+        return KYN_OK;
+    });
+}
+
+int kyn_debug_get_launch(kyn_system s, int* fused_workgroups, int* element_workgroups) {
+    return guarded([&] {
+        if (!s) throw KynError(KYN_ERR_INVALID, "null system");
+        if (fused_workgroups) *fused_workgroups = s->S.num_fused_work;
+        if (element_workgroups) *element_workgroups = s->S.elem_split && s->S.precision == 0 ? 3 : 1;
+        return KYN_OK;
+    });
+}
+
+int kyn_debug_set_fused_workgroups(kyn_system s, int per_model) {
+    return guarded([&] {
+        if (!s || per_model < 1) throw KynError(KYN_ERR_INVALID, "a model's step takes at least one workgroup");
+        std::vector<int> work, blocks(s->num_models, 0);
+        for (size_t g = 0; g < s->fused_work.size(); g += 2) ++blocks[s->fused_work[g]];
+        for (size_t g = 0; g < s->fused_work.size(); g += 2)
+            if (s->fused_work[g + 1] >= blocks[s->fused_work[g]] - per_model)
+                work.insert(work.end(), {s->fused_work[g], s->fused_work[g + 1]});
+        s->S.fused_work = s->arena.up(work);
+        s->S.num_fused_work = static_cast<int>(work.size() / 2);
+        s->graph_ready = false;  // the captured step holds the kernel arguments
         return KYN_OK;
     });
 }

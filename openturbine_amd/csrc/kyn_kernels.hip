@@ -1833,15 +1833,15 @@ __device__ __forceinline__ void apply_schedule_model(const DevSys& S, int m, Min
         }
 }
 
-// After a step: the schedule's next row, and the split launch's ticket and exchange slots cleared
-// for the next step (thread per block; the slots its model's iterations used, all of them after a
-// wait that gave up).
+// After a step: the schedule's next row, and the split launch's ticket, claims and exchange slots
+// cleared for the next step (thread per block; the slots its model's iterations used, all of them
+// after a wait that gave up).
 __global__ void k_advance_slot(DevSys S) {
     const int g = blockIdx.x * blockDim.x + threadIdx.x;
     if (g == 0 && S.sched_steps > 0) *S.sched_slot += 1;
-    if (S.fused_ticket == nullptr) return;
-    if (g == 0) *S.fused_ticket = 0;
-    if (g < S.num_blocks) {
+    if (g == 0 && S.fused_ticket != nullptr) *S.fused_ticket = 0;
+    if (S.fused_claim != nullptr && g < S.num_blocks) {
+        S.fused_claim[g] = 0;
         const int used = *S.dev_error != 0 ? S.p.max_iter : S.model_iters[S.block_model[g]];
         for (int k = 0; k < used; ++k) S.fused_xch[(size_t)g * S.p.max_iter + k] = kXchEmpty;
     }
@@ -2258,47 +2258,52 @@ __device__ __forceinline__ void factor_solve_uncondition(const DevSys& S, int b,
 }
 
 // ---------------------------------------------------------------------------------------
-// Fused form: one launch per time step, one workgroup per model, or one per block of a model
-// where the models alone leave the chip idle (the launch list fused_work, built at setup).
+// Fused form: one launch per time step, one workgroup per model, or one per block where the models
+// alone leave the chip idle (the launch list fused_work, built at setup).
 //
-// Split models: a model's blocks share nothing but the convergence error, so each block's Newton
-// loop runs in a workgroup of its own, and per iteration the workgroups exchange one number: each
-// stores its block's error sum into the slot (block, iteration) and reads the others', summed
-// in block order, so every workgroup takes the same decision and all results are those of the
-// unsplit form bit for bit.  The number is the only thing one reads of another, so the exchange is
-// a relaxed device-scope store and load of one 64-bit word (an empty slot holds kXchEmpty).
-// Workgroups take their list entry by ticket in the order they start and a model's entries are
-// consecutive: whoever waits, the earliest unfinished model's workgroups are all running or the
-// next to start, so every wait ends (the host splits only models with no more blocks than the
-// chip has CUs).  The wait is bounded all the same.
+// Split launch: a model's blocks share nothing but the convergence error, so their Newton loops run
+// in different workgroups, and per iteration the workgroups exchange one number per block: its
+// error sum, stored into the slot (block, iteration); every workgroup of the model reads them all,
+// summed in block order, so all take the same decision and all results are those of the unsplit
+// form bit for bit.  The number is the only thing one reads of another, so the exchange is a relaxed
+// device-scope store and load of one 64-bit word (an empty slot holds kXchEmpty).
+//
+// Every wait ends whatever share of the chip the launch gets (other streams' kernels, masked CUs,
+// workgroups started in any order), because a block waited for has a running workgroup: each claims
+// its block as it starts (and ends at once if another has it), and one that has waited kLatePolls
+// in the first iteration claims blocks of its model that nobody has, runs them beside its own from
+// then on, and waits again.  With room for one workgroup of a model, that one runs the unsplit
+// form.  kLatePolls is ~3 ms, longer than a block waits for a place where this launch has the chip
+// to itself (a claim right after a workgroup's own block: 256 FP64 rotors 2.27 -> 2.43 ms, 96 1.20 ->
+// 1.30, since a block taken over stays in line behind another for the whole step).
 // Measured, us per step unsplit / split: one 3-blade rotor, FP64 2597 / 1061, FP32 1989 / 834; 96
 // rotors of mixed blade sizes, FP64 2940 / 1442, FP32 2303 / 942.
 // ---------------------------------------------------------------------------------------
-// Whether the workgroup of a split model's block owns a node: its block's, and the first
-// block's workgroup also the nodes of no block.
-__device__ __forceinline__ bool owns_node(const DevSys& S, int node, int part, int block) {
-    const int nb = S.node_block[node];
-    return nb < 0 ? part == 0 : nb == block;
+// Publishes one block's error sum of one iteration.
+__device__ __forceinline__ void publish_err_sum(const DevSys& S, int b, int iter, double own) {
+    if (threadIdx.x == 0) {
+        unsigned long long w = (unsigned long long)__double_as_longlong(own);
+        if (w == kXchEmpty) w = 0x7ff8000000000000ull;  // any NaN does
+        __hip_atomic_store(S.fused_xch + (size_t)b * S.p.max_iter + iter, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
 }
 
-// Publishes this block's error sum of one iteration and returns the model's, through red[0]; false
-// when the wait for the other blocks gave up.
-__device__ __forceinline__ bool exchange_err_sum(const DevSys& S, int b0, int nb, int b, int iter, double own, double* red,
-                                                 double& sum) {
+// Waits for the error sums of all the model's blocks in one iteration.  kPeersDone: their sum, through
+// red[0], is in `sum`; kPeersLate: still waiting after `late` polls; kPeersGaveUp: after the
+// bound.
+constexpr int kPeersDone = 0, kPeersLate = 1, kPeersGaveUp = 2;
+__device__ __forceinline__ int collect_err_sum(const DevSys& S, int b0, int nb, int iter, int late, double* red,
+                                               double& sum) {
     const int t = threadIdx.x;
     if (t < 64) {
         unsigned long long* slot = S.fused_xch + iter;
-        if (t == 0) {
-            unsigned long long w = (unsigned long long)__double_as_longlong(own);
-            if (w == kXchEmpty) w = 0x7ff8000000000000ull;  // any NaN does
-            __hip_atomic_store(slot + (size_t)b * S.p.max_iter, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
         unsigned long long w = t < nb ? kXchEmpty : 0;
         int polls = 0;
         for (;; ++polls) {
             if (w == kXchEmpty)
                 w = __hip_atomic_load(slot + (size_t)(b0 + t) * S.p.max_iter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             if (!__any(w == kXchEmpty)) break;
+            if (polls >= late) break;
             if (polls >= kPeerWaitLimit) {
                 if (t == 0) __hip_atomic_fetch_or(S.dev_error, kDevErrPeerWait, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 break;
@@ -2310,12 +2315,22 @@ __device__ __forceinline__ bool exchange_err_sum(const DevSys& S, int b0, int nb
         for (int k = 0; k < nb; ++k) acc += rdlane(v, k);
         if (t == 0) {
             red[0] = acc;
-            red[1] = polls < kPeerWaitLimit ? 1. : 0.;
+            red[1] = polls >= late ? kPeersLate : polls >= kPeerWaitLimit ? kPeersGaveUp : kPeersDone;
         }
     }
     __syncthreads();
     sum = red[0];
-    return red[1] != 0.;
+    return __builtin_amdgcn_readfirstlane((int)red[1]);
+}
+
+// Claims the first of the model's blocks [k, k1) that no workgroup has; k1 if there is none.
+__device__ __forceinline__ int claim_block(const DevSys& S, int mb0, int k, int k1, int* misc) {
+    if (threadIdx.x == 0) {
+        while (k < k1 && atomicCAS(S.fused_claim + mb0 + k, 0, 1) != 0) ++k;
+        misc[0] = k;
+    }
+    __syncthreads();
+    return __builtin_amdgcn_readfirstlane(misc[0]);
 }
 
 // The kernel's first argument, read anew from the kernel-argument segment: what is loaded through
@@ -2328,33 +2343,10 @@ __device__ __forceinline__ const DevSys& sys_args() {
     return *(const DevSys*)p;
 }
 
-template <typename TT>
-__device__ __forceinline__ void fused_step_body(int Nm, int Qm, int nm) {
-    extern __shared__ __align__(16) char sm[];
-    const DevSys& S = sys_args();
-    const Lay L = make_layout(Nm, Qm, nm, S.max_block_cons, S.refine_sweeps > 0, (int)sizeof(TT), true);
+// Inputs, PredictNextState and ResetConstraints (step.hpp:49-50) of the nodes mine() picks.
+template <typename Mine>
+__device__ __forceinline__ void fused_begin(const DevSys& S, int m, Mine mine) {
     const int t = threadIdx.x;
-    double* red = reinterpret_cast<double*>(sm + L.red);
-    int* misc = reinterpret_cast<int*>(sm + L.misc);
-    double* rhs = reinterpret_cast<double*>(sm + L.rhs);
-    double* xs = reinterpret_cast<double*>(sm + L.xs);
-    double* xs2 = reinterpret_cast<double*>(sm + L.xs2);
-    int* piv = reinterpret_cast<int*>(sm + L.piv);
-    TT* A = reinterpret_cast<TT*>(sm + L.A);
-
-    int g = blockIdx.x;
-    if (S.fused_ticket != nullptr) {  // uniform
-        if (t == 0) misc[0] = atomicAdd(S.fused_ticket, 1);
-        __syncthreads();
-        g = __builtin_amdgcn_readfirstlane(misc[0]);
-    }
-    const int m = S.fused_work[2 * g], part = S.fused_work[2 * g + 1];  // part: block within the model, -1: all
-    const int mb0 = S.model_block_begin[m], mb1 = S.model_block_end[m];
-    const int b0 = part < 0 ? mb0 : mb0 + part, b1 = part < 0 ? mb1 : b0 + 1;
-    const bool lead = part <= 0;  // writes the model's bookkeeping
-    auto mine = [&](int node) { return part < 0 || owns_node(S, node, part, b0); };
-
-    // inputs, PredictNextState, ResetConstraints (step.hpp:49-50)
     apply_schedule_model(S, m, mine);
     __syncthreads();
     for (int node = S.model_node_begin[m] + t; node < S.model_node_end[m]; node += blockDim.x)
@@ -2367,7 +2359,79 @@ __device__ __forceinline__ void fused_step_body(int Nm, int Qm, int nm) {
                 S.con_sys_res[c * 6 + k] = 0.;
             }
     __syncthreads();
+}
 
+// One block's share of a Newton iteration; returns its error sum.
+template <typename TT>
+__device__ __forceinline__ double fused_block_iteration(char* sm, const Lay& L, int m, int b, double err_prev) {
+    const int t = threadIdx.x;
+    double* rhs = reinterpret_cast<double*>(sm + L.rhs);
+    double* xs = reinterpret_cast<double*>(sm + L.xs);
+    double* xs2 = reinterpret_cast<double*>(sm + L.xs2);
+    int* piv = reinterpret_cast<int*>(sm + L.piv);
+    TT* A = reinterpret_cast<TT*>(sm + L.A);
+    KYN_PHASE_MARK(0);
+    int n;
+    {
+        const DevSys& S = sys_args();
+        n = S.block_n[b];
+        const int e = S.block_elems[S.block_elem_begin[b]];
+        // every system row starts at -f (a node outside the element, e.g. a massless hub,
+        // takes only its load and constraint terms); the element rows are then written as
+        // -f + R after the element phase's first barrier
+        for (int i = t; i < S.block_nsys[b]; i += blockDim.x)
+            rhs[i] = -S.f[S.block_nodes[S.block_node_begin[b] + i / 6] * 6 + i % 6];
+        element_phase<TT, true>(S, e, sm, L, n, nullptr, nullptr, m);
+    }
+    KYN_PHASE_MARK(5);
+    block_constraints<TT>(sys_args(), b, sm, L);
+    condition_rhs(sys_args(), b, rhs);
+    KYN_PHASE_MARK(6);
+    {
+        const DevSys& S = sys_args();
+        // FP64 refinement of the FP32 solve where it decides the final state: the Newton
+        // increments contract by ~20x per iteration, so a solve error matters only in the
+        // last iterations, whose predecessors' errors are small (an inexact-Newton forcing
+        // rule)
+        const bool refine_now = S.refine_sweeps > 0 && (S.refine_err_bound <= 0. || err_prev < S.refine_err_bound);
+        // unfactored copy for refinement: row-major, row stride (n + 3) & ~3, at the block's own offset
+        TT* Ac = (S.Acopy != nullptr && refine_now) ? reinterpret_cast<TT*>(S.Acopy) + S.block_C_off[b] : nullptr;
+        factor_solve_uncondition<TT>(S, b, A, Ac, L.lda, piv, rhs, xs, xs2, sm, L);
+    }
+    KYN_PHASE_MARK(10);
+    const double sum = block_error_and_update(sys_args(), b, xs, reinterpret_cast<double*>(sm + L.red));
+    KYN_PHASE_MARK(11);
+    return sum;
+}
+
+// Step epilogue of the nodes mine() picks (on convergence), and the model's bookkeeping.
+template <typename Mine>
+__device__ __forceinline__ void fused_end(const DevSys& S, int m, int converged, int iter, bool lead, Mine mine) {
+    const int t = threadIdx.x;
+    if (converged) {
+        for (int node = S.model_node_begin[m] + t; node < S.model_node_end[m]; node += blockDim.x)
+            if (mine(node)) epilogue_node(S, node);
+        for (int c = S.model_con_begin[m] + t; c < S.model_con_end[m]; c += blockDim.x)
+            if (mine(S.con_target[c])) constraint_output(S, c);
+    }
+    if (t == 0 && lead) {
+        S.model_status[m] = converged ? 0 : 1;
+        S.model_iters[m] = iter;
+        S.model_active[m] = 0;
+        S.model_iter_total[m] += iter;
+        S.model_fail_total[m] += converged ? 0 : 1;
+    }
+}
+
+// A workgroup per model.
+template <typename TT>
+__device__ __forceinline__ void fused_step_body(int Nm, int Qm, int nm) {
+    extern __shared__ __align__(16) char sm[];
+    const DevSys& S = sys_args();
+    const Lay L = make_layout(Nm, Qm, nm, S.max_block_cons, S.refine_sweeps > 0, (int)sizeof(TT), true);
+    const int m = S.fused_work[2 * blockIdx.x];
+    const auto all = [](int) { return true; };
+    fused_begin(S, m, all);
     const double ndofs = (double)S.model_ndofs[m];
     const int max_iter = S.p.max_iter;
     int converged = 0;
@@ -2375,46 +2439,11 @@ __device__ __forceinline__ void fused_step_body(int Nm, int Qm, int nm) {
     double err_prev = __builtin_inf();  // convergence error of the previous Newton iteration
     for (; iter < max_iter; ++iter) {
         double err_sum = 0.;
-        for (int b = b0; b < b1; ++b) {
-            KYN_PHASE_MARK(0);
-            int n;
-            {
-                const DevSys& S = sys_args();
-                n = S.block_n[b];
-                const int e = S.block_elems[S.block_elem_begin[b]];
-                // every system row starts at -f (a node outside the element, e.g. a massless hub,
-                // takes only its load and constraint terms); the element rows are then written as
-                // -f + R after the element phase's first barrier
-                for (int i = t; i < S.block_nsys[b]; i += blockDim.x)
-                    rhs[i] = -S.f[S.block_nodes[S.block_node_begin[b] + i / 6] * 6 + i % 6];
-                element_phase<TT, true>(S, e, sm, L, n, nullptr, nullptr, m);
-            }
-            KYN_PHASE_MARK(5);
-            block_constraints<TT>(sys_args(), b, sm, L);
-            condition_rhs(sys_args(), b, rhs);
-            KYN_PHASE_MARK(6);
-            {
-                const DevSys& S = sys_args();
-                // FP64 refinement of the FP32 solve where it decides the final state: the Newton
-                // increments contract by ~20x per iteration, so a solve error matters only in the
-                // last iterations, whose predecessors' errors are small (an inexact-Newton forcing
-                // rule)
-                const bool refine_now =
-                    S.refine_sweeps > 0 && (S.refine_err_bound <= 0. || err_prev < S.refine_err_bound);
-                // unfactored copy for refinement: row-major, row stride (n + 3) & ~3, at the block's own offset
-                TT* Ac =
-                    (S.Acopy != nullptr && refine_now) ? reinterpret_cast<TT*>(S.Acopy) + S.block_C_off[b] : nullptr;
-                factor_solve_uncondition<TT>(S, b, A, Ac, L.lda, piv, rhs, xs, xs2, sm, L);
-            }
-            KYN_PHASE_MARK(10);
-            err_sum += block_error_and_update(sys_args(), b, xs, red);
-            KYN_PHASE_MARK(11);
-        }
-        const DevSys& S = sys_args();
-        if (part >= 0 && !exchange_err_sum(S, mb0, mb1 - mb0, b0, iter, err_sum, red, err_sum)) break;
+        for (int b = S.model_block_begin[m]; b < S.model_block_end[m]; ++b)
+            err_sum += fused_block_iteration<TT>(sm, L, m, b, err_prev);
         const double err = sqrt(err_sum / ndofs);
         err_prev = err;
-        if (t == 0 && lead) S.err_hist[(size_t)m * max_iter + iter] = err;
+        if (threadIdx.x == 0) sys_args().err_hist[(size_t)m * max_iter + iter] = err;
         // the reference's loop test `err > 1.` (step.hpp:54): a NaN error also ends the loop,
         // and the step then counts as converged
         if (!(err > 1.)) {
@@ -2423,22 +2452,81 @@ __device__ __forceinline__ void fused_step_body(int Nm, int Qm, int nm) {
             break;
         }
     }
+    fused_end(sys_args(), m, converged, iter, true, all);
+}
+
+// A workgroup per list entry of a split launch.
+template <typename TT>
+__device__ __forceinline__ void fused_split_body(int Nm, int Qm, int nm) {
+    extern __shared__ __align__(16) char sm[];
+    const DevSys& S = sys_args();
+    const Lay L = make_layout(Nm, Qm, nm, S.max_block_cons, S.refine_sweeps > 0, (int)sizeof(TT), true);
+    const int t = threadIdx.x;
+    double* red = reinterpret_cast<double*>(sm + L.red);
+    int* misc = reinterpret_cast<int*>(sm + L.misc);
+    int g = blockIdx.x;
+    if (S.fused_ticket != nullptr) {  // uniform
+        if (t == 0) misc[1] = atomicAdd(S.fused_ticket, 1);
+        __syncthreads();
+        g = __builtin_amdgcn_readfirstlane(misc[1]);
+    }
+    const int m = S.fused_work[2 * g], k0 = S.fused_work[2 * g + 1];
+    const int mb0 = S.model_block_begin[m], nb = S.model_block_end[m] - mb0;
+    if (claim_block(S, mb0, k0, k0 + 1, misc) != k0) return;
+    unsigned long long own = 0;  // the model's blocks run here
+    const auto begin = [&](int k) {  // the block's nodes; with the model's first block also those of no block
+        own |= 1ull << k;
+        const DevSys& S = sys_args();
+        fused_begin(S, m, [&](int node) {
+            const int nbk = S.node_block[node];
+            return nbk < 0 ? k == 0 : nbk == mb0 + k;
+        });
+    };
+    begin(k0);
+    const double ndofs = (double)S.model_ndofs[m];
+    const int max_iter = S.p.max_iter;
+    int converged = 0;
+    int iter = 0;
+    double err_prev = __builtin_inf();
+    for (; iter < max_iter; ++iter) {
+        double err_sum;
+        int code = kPeersDone;
+        int late = iter == 0 ? kLatePolls : INT_MAX;
+        int k = iter == 0 ? k0 : __builtin_ctzll(own);
+        for (;;) {
+            if (k < nb) {
+                const double block_err = fused_block_iteration<TT>(sm, L, m, mb0 + k, err_prev);
+                publish_err_sum(sys_args(), mb0 + k, iter, block_err);
+                const unsigned long long rest = iter == 0 ? 0 : own >> k >> 1;
+                if (rest != 0) {
+                    k += 1 + __builtin_ctzll(rest);
+                    continue;
+                }
+            }
+            code = collect_err_sum(sys_args(), mb0, nb, iter, late, red, err_sum);
+            if (code != kPeersLate) break;
+            k = claim_block(sys_args(), mb0, 0, nb, misc);
+            if (k < nb)
+                begin(k);
+            else
+                late = INT_MAX;  // every block has its workgroup
+        }
+        if (code == kPeersGaveUp) break;
+        const double err = sqrt(err_sum / ndofs);
+        err_prev = err;
+        if (t == 0 && (own & 1)) sys_args().err_hist[(size_t)m * max_iter + iter] = err;
+        if (!(err > 1.)) {  // as in fused_step_body
+            converged = 1;
+            ++iter;
+            break;
+        }
+    }
     {
         const DevSys& S = sys_args();
-        auto mine = [&](int node) { return part < 0 || owns_node(S, node, part, b0); };
-        if (converged) {
-            for (int node = S.model_node_begin[m] + t; node < S.model_node_end[m]; node += blockDim.x)
-                if (mine(node)) epilogue_node(S, node);
-            for (int c = S.model_con_begin[m] + t; c < S.model_con_end[m]; c += blockDim.x)
-                if (mine(S.con_target[c])) constraint_output(S, c);
-        }
-        if (t == 0 && lead) {
-            S.model_status[m] = converged ? 0 : 1;
-            S.model_iters[m] = iter;
-            S.model_active[m] = 0;
-            S.model_iter_total[m] += iter;
-            S.model_fail_total[m] += converged ? 0 : 1;
-        }
+        fused_end(S, m, converged, iter, (own & 1) != 0, [&](int node) {
+            const int nbk = S.node_block[node];
+            return ((own >> (nbk < 0 ? 0 : nbk - mb0)) & 1) != 0;
+        });
     }
 }
 
@@ -2446,10 +2534,16 @@ __device__ __forceinline__ void fused_step_body(int Nm, int Qm, int nm) {
 __global__ void __launch_bounds__(kThreads) k_fused_step_f64(DevSys S, int Nm, int Qm, int nm) {
     fused_step_body<double>(Nm, Qm, nm);
 }
+__global__ void __launch_bounds__(kThreads) k_fused_split_f64(DevSys S, int Nm, int Qm, int nm) {
+    fused_split_body<double>(Nm, Qm, nm);
+}
 // FP32 tangent: blocks up to 143 dofs fit in 80 KB, so two workgroups share a CU (registers
 // capped at 256 per lane for that).
 __global__ void __launch_bounds__(kThreads, 2) k_fused_step_f32(DevSys S, int Nm, int Qm, int nm) {
     fused_step_body<float>(Nm, Qm, nm);
+}
+__global__ void __launch_bounds__(kThreads, 2) k_fused_split_f32(DevSys S, int Nm, int Qm, int nm) {
+    fused_split_body<float>(Nm, Qm, nm);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -3560,6 +3654,10 @@ hipError_t set_lds_limits(size_t bytes) {
     if (e != hipSuccess) return e;
     e = hipFuncSetAttribute((const void*)k_fused_step_f32, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
     if (e != hipSuccess) return e;
+    e = hipFuncSetAttribute((const void*)k_fused_split_f64, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+    if (e != hipSuccess) return e;
+    e = hipFuncSetAttribute((const void*)k_fused_split_f32, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+    if (e != hipSuccess) return e;
     e = hipFuncSetAttribute((const void*)k_plain_element, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
     if (e != hipSuccess) return e;
     e = hipFuncSetAttribute((const void*)k_plain_element_split, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
@@ -3581,10 +3679,9 @@ hipError_t set_lds_limits(size_t bytes) {
 
 void launch_fused_step(const DevSys& S, int Nm, int Qm, int nm, hipStream_t st) {
     const size_t lds = fused_lds_bytes(Nm, Qm, nm, S.max_block_cons, S.refine_sweeps, S.precision);
-    if (S.precision)
-        hipLaunchKernelGGL(k_fused_step_f32, dim3(S.num_fused_work), dim3(kThreads), lds, st, S, Nm, Qm, nm);
-    else
-        hipLaunchKernelGGL(k_fused_step_f64, dim3(S.num_fused_work), dim3(kThreads), lds, st, S, Nm, Qm, nm);
+    const auto k = S.fused_claim != nullptr ? (S.precision ? k_fused_split_f32 : k_fused_split_f64)
+                                             : (S.precision ? k_fused_step_f32 : k_fused_step_f64);
+    hipLaunchKernelGGL(k, dim3(S.num_fused_work), dim3(kThreads), lds, st, S, Nm, Qm, nm);
 }
 // ---------------------------------------------------------------------------------------
 // Element-terms scratch of the no-allocation entry point: one element's residual [N][6] and
@@ -3621,7 +3718,7 @@ void launch_element_terms(const DevSys& S, int Nm, int Qm, int e, double* res, d
 }
 
 void launch_advance_slot(const DevSys& S, hipStream_t st) {
-    const bool split = S.fused_ticket != nullptr;
+    const bool split = S.fused_claim != nullptr;
     hipLaunchKernelGGL(k_advance_slot, dim3(split ? (S.num_blocks + 63) / 64 : 1), dim3(64), 0, st, S);
 }
 void launch_plain_predict(const DevSys& S, hipStream_t st) {

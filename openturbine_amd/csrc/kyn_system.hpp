@@ -71,11 +71,12 @@ struct DevSys {
     const int* model_ndofs;
     const double* model_gravity;  // [m][3]
     const int* model_load_begin;  // into sched_load_nodes (sorted by node), [m+1]
-    // ---- fused launch: workgroup g runs fused_work[2 g] = model (costliest first), fused_work[2 g + 1]
-    //      = the one block of it to run, counted from the model's first, or -1 for all of them
+    // ---- fused launch: workgroup g runs fused_work[2 g] = model (costliest first) and, in a split
+    //      launch, starts with its block fused_work[2 g + 1], counted from the model's first
     const int* fused_work;
     int num_fused_work;
-    int* fused_ticket;              // split launch (else null): list entries taken by started workgroups
+    int* fused_ticket;              // split launch of more workgroups than places (else null): see host
+    int* fused_claim;               // split launch (else null): [block] 1 once a workgroup runs it in this step
     unsigned long long* fused_xch;  // split launch: [block][max_iter] error sums, kXchEmpty until stored
 
     // ---- blocks
@@ -255,6 +256,7 @@ constexpr int kDevErrLuWait = 1;
 constexpr unsigned long long kXchEmpty = ~0ull;
 constexpr int kPeerWaitLimit = 1 << 26;
 constexpr int kDevErrPeerWait = 2;
-constexpr int kMaxSplitBlocks = 64;  // blocks of a split model: one lane each polls a block's slot
+constexpr int kMaxSplitBlocks = 64;  // blocks per model of a split launch: one lane each polls a block's slot
+constexpr int kLatePolls = 1 << 14;  // split launch: polls before a workgroup looks for blocks that have none
 
 }  // namespace kyn
