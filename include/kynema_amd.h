@@ -209,6 +209,9 @@ int kyn_debug_assemble(kyn_system s);
  * step returns KYN_ERR_HIP; polls < 0 gives up at the first wait (tests of that error path).
  * No counterpart in the reference (its LU runs on the host). */
 int kyn_debug_set_wait_limit(kyn_system s, int polls);
+/* The same for the wait between the workgroups of a split fused step (each waits once per Newton
+ * iteration for its model's other blocks; default 1 << 24 polls, seconds). */
+int kyn_debug_set_peer_wait_limit(kyn_system s, int polls);
 /* Engine of the FP32 tangent's node-pair contraction per element node count N: bit N of `mask`
  * set selects the matrix cores, clear the VALU register tile.  The default is the compiled-in
  * tuning table (openturbine_amd/autotune.py); this call overrides it (the autotuner, tests).

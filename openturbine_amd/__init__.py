@@ -172,6 +172,7 @@ class KynLib:
         L.kyn_read_restart.argtypes = [C.c_void_p, C.c_size_t, C.POINTER(C.c_ubyte), C.c_size_t]
         L.kyn_debug_assemble.argtypes = [C.c_void_p]
         L.kyn_debug_set_wait_limit.argtypes = [C.c_void_p, C.c_int]
+        L.kyn_debug_set_peer_wait_limit.argtypes = [C.c_void_p, C.c_int]
         L.kyn_debug_set_contraction_mask.argtypes = [C.c_void_p, C.c_uint]
         L.kyn_debug_get_launch.argtypes = [C.c_void_p, C.POINTER(C.c_int), C.POINTER(C.c_int)]
         L.kyn_debug_set_fused_workgroups.argtypes = [C.c_void_p, C.c_int]

@@ -998,8 +998,9 @@ void check_device_errors(kyn_system_s* s) {
     const int zero = 0;
     hip_check(hipMemcpy(s->S.dev_error, &zero, sizeof(int), hipMemcpyHostToDevice), "H2D");
     if (!(flags & kyn::kDevErrLuWait))
-        throw KynError(KYN_ERR_HIP, "a workgroup of the fused step gave up waiting for the other blocks of its model; "
-                                    "the step's results are invalid");
+        throw KynError(KYN_ERR_HIP, "a workgroup of the fused step gave up waiting for the other blocks of its model "
+                                    "(bound " + std::to_string(s->S.peer_wait_limit) +
+                                    " polls); the step's results are invalid");
     throw KynError(KYN_ERR_HIP, "a wave of the blocked LU gave up waiting on its look-ahead counter "
                                 "(bound " + std::to_string(s->S.lu_wait_limit) + " polls); the step's results are invalid");
 }
@@ -1764,6 +1765,7 @@ kyn_system kyn_system_create(const kyn_model* models, size_t num_models, const k
         S.sched_slot = Ar.zeros<int>(1);
         S.dev_error = Ar.zeros<int>(1);
         S.lu_wait_limit = kyn::kLuWaitLimitDefault;
+        S.peer_wait_limit = kyn::kPeerWaitLimitDefault;
         S.sched_steps = 0;
 
         // ---- host copies of the layout
@@ -2209,6 +2211,15 @@ int kyn_read_restart(kyn_system s, size_t model, const unsigned char* in, size_t
             hip_check(hipMemcpy(p + n0 * w, in + off, n * w * sizeof(double), hipMemcpyHostToDevice), "H2D");
             off += n * w * sizeof(double);
         }
+        return KYN_OK;
+    });
+}
+
+int kyn_debug_set_peer_wait_limit(kyn_system s, int polls) {
+    return guarded([&] {
+        if (!s) throw KynError(KYN_ERR_INVALID, "null system");
+        s->S.peer_wait_limit = polls;
+        s->graph_ready = false;  // the captured step holds the kernel arguments
         return KYN_OK;
     });
 }

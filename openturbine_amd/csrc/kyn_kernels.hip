@@ -2273,7 +2273,7 @@ __device__ __forceinline__ void factor_solve_uncondition(const DevSys& S, int b,
 // its block as it starts (and ends at once if another has it), and one that has waited kLatePolls
 // in the first iteration claims blocks of its model that nobody has, runs them beside its own from
 // then on, and waits again.  With room for one workgroup of a model, that one runs the unsplit
-// form.  kLatePolls is ~3 ms, longer than a block waits for a place where this launch has the chip
+// form.  kLatePolls is 2.3 ms, longer than a block waits for a place where this launch has the chip
 // to itself (a claim right after a workgroup's own block: 256 FP64 rotors 2.27 -> 2.43 ms, 96 1.20 ->
 // 1.30, since a block taken over stays in line behind another for the whole step).
 // Measured, us per step unsplit / split: one 3-blade rotor, FP64 2597 / 1061, FP32 1989 / 834; 96
@@ -2289,8 +2289,9 @@ __device__ __forceinline__ void publish_err_sum(const DevSys& S, int b, int iter
 }
 
 // Waits for the error sums of all the model's blocks in one iteration.  kPeersDone: their sum, through
-// red[0], is in `sum`; kPeersLate: still waiting after `late` polls; kPeersGaveUp: after the
-// bound.
+// red[0], is in `sum`; kPeersLate: still waiting after `late` polls; kPeersGaveUp: after
+// peer_wait_limit polls, or because another workgroup of this step, or of an earlier one not yet
+// reported, gave up (looked at every kErrorPolls polls): that one publishes nothing more.
 constexpr int kPeersDone = 0, kPeersLate = 1, kPeersGaveUp = 2;
 __device__ __forceinline__ int collect_err_sum(const DevSys& S, int b0, int nb, int iter, int late, double* red,
                                                double& sum) {
@@ -2299,12 +2300,16 @@ __device__ __forceinline__ int collect_err_sum(const DevSys& S, int b0, int nb, 
         unsigned long long* slot = S.fused_xch + iter;
         unsigned long long w = t < nb ? kXchEmpty : 0;
         int polls = 0;
+        bool gave_up = false;
         for (;; ++polls) {
             if (w == kXchEmpty)
                 w = __hip_atomic_load(slot + (size_t)(b0 + t) * S.p.max_iter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             if (!__any(w == kXchEmpty)) break;
             if (polls >= late) break;
-            if (polls >= kPeerWaitLimit) {
+            gave_up = polls >= S.peer_wait_limit ||
+                      (polls % kErrorPolls == kErrorPolls - 1 &&
+                       (__hip_atomic_load(S.dev_error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & kDevErrPeerWait) != 0);
+            if (gave_up) {
                 if (t == 0) __hip_atomic_fetch_or(S.dev_error, kDevErrPeerWait, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 break;
             }
@@ -2315,7 +2320,7 @@ __device__ __forceinline__ int collect_err_sum(const DevSys& S, int b0, int nb, 
         for (int k = 0; k < nb; ++k) acc += rdlane(v, k);
         if (t == 0) {
             red[0] = acc;
-            red[1] = polls >= late ? kPeersLate : polls >= kPeerWaitLimit ? kPeersGaveUp : kPeersDone;
+            red[1] = gave_up ? kPeersGaveUp : polls >= late ? kPeersLate : kPeersDone;
         }
     }
     __syncthreads();
@@ -2494,24 +2499,23 @@ __device__ __forceinline__ void fused_split_body(int Nm, int Qm, int nm) {
         int late = iter == 0 ? kLatePolls : INT_MAX;
         int k = iter == 0 ? k0 : __builtin_ctzll(own);
         for (;;) {
+            const double block_err = k < nb ? fused_block_iteration<TT>(sm, L, m, mb0 + k, err_prev) : 0.;
+            const DevSys& S = sys_args();
             if (k < nb) {
-                const double block_err = fused_block_iteration<TT>(sm, L, m, mb0 + k, err_prev);
-                publish_err_sum(sys_args(), mb0 + k, iter, block_err);
+                publish_err_sum(S, mb0 + k, iter, block_err);
                 const unsigned long long rest = iter == 0 ? 0 : own >> k >> 1;
                 if (rest != 0) {
                     k += 1 + __builtin_ctzll(rest);
                     continue;
                 }
             }
-            code = collect_err_sum(sys_args(), mb0, nb, iter, late, red, err_sum);
+            code = collect_err_sum(S, mb0, nb, iter, late, red, err_sum);
             if (code != kPeersLate) break;
-            k = claim_block(sys_args(), mb0, 0, nb, misc);
-            if (k < nb)
-                begin(k);
-            else
-                late = INT_MAX;  // every block has its workgroup
+            k = claim_block(S, mb0, 0, nb, misc);
+            late = k < nb ? 0 : INT_MAX;  // (waited long enough for a start; every block has its workgroup)
+            if (k < nb) begin(k);
         }
-        if (code == kPeersGaveUp) break;
+        if (code == kPeersGaveUp) return;  // the step is an error, none of its numbers count
         const double err = sqrt(err_sum / ndofs);
         err_prev = err;
         if (t == 0 && (own & 1)) sys_args().err_hist[(size_t)m * max_iter + iter] = err;

@@ -245,18 +245,22 @@ struct DevSys {
     //      gives up after lu_wait_limit polls (< 0: at its first wait), sets bit 0 of
     //      dev_error and goes on, so the kernel still ends; the host reports the flag
     int lu_wait_limit;
+    //      likewise a workgroup of the split fused launch that waits for its model's others
+    //      (peer_wait_limit, bit 1): it leaves the step, and so do those that wait for it
+    int peer_wait_limit;
     int* dev_error;
 };
 
 constexpr int kLuWaitLimitDefault = 1 << 20;  // polls of ~64 cycles: ~28 ms at 2.4 GHz
 constexpr int kDevErrLuWait = 1;
-// split fused launch: an exchange slot nobody has stored to (a NaN that no error sum is stored
-// as), and the polls (~0.2 us each) a workgroup waits for its model's other blocks: seconds, since
-// they may not have started behind another stream's kernels
+// split fused launch: an exchange slot nobody has stored to (a NaN that no error sum is stored as), and
+// the polls (0.28 us each) a workgroup waits for its model's other blocks, which are all running
+// when it counts: 4.7 s, against milliseconds for a Newton iteration
 constexpr unsigned long long kXchEmpty = ~0ull;
-constexpr int kPeerWaitLimit = 1 << 26;
+constexpr int kPeerWaitLimitDefault = 1 << 24;
+constexpr int kErrorPolls = 1 << 12;  // polls between looks at dev_error (1.1 ms)
 constexpr int kDevErrPeerWait = 2;
 constexpr int kMaxSplitBlocks = 64;  // blocks per model of a split launch: one lane each polls a block's slot
-constexpr int kLatePolls = 1 << 14;  // split launch: polls before a workgroup looks for blocks that have none
+constexpr int kLatePolls = 1 << 13;  // split launch: polls before a workgroup looks for blocks that have none
 
 }  // namespace kyn
