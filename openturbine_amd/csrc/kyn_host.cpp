@@ -1304,7 +1304,8 @@ kyn_system kyn_system_create(const kyn_model* models, size_t num_models, const k
                 most_blocks = std::max(most_blocks, B.model_block_end[m] - B.model_block_begin[m]);
             }
             const bool split = sys->exec_mode == KYN_EXEC_FUSED && fused_split_models(num_models, cus, S.precision != 0) &&
-                               least_blocks >= 1 && most_blocks >= 2 && most_blocks <= kyn::kMaxSplitBlocks;
+                               least_blocks >= 1 && most_blocks >= 2 && most_blocks <= kyn::kMaxSplitBlocks &&
+                               S.p.max_iter <= kyn::kMaxSplitIters;
             for (int m : order) {
                 const int nb = split ? B.model_block_end[m] - B.model_block_begin[m] : 1;
                 for (int k = 0; k < nb; ++k) sys->fused_work.insert(sys->fused_work.end(), {m, k});

@@ -261,6 +261,7 @@ constexpr int kPeerWaitLimitDefault = 1 << 24;
 constexpr int kErrorPolls = 1 << 12;  // polls between looks at dev_error (1.1 ms)
 constexpr int kDevErrPeerWait = 2;
 constexpr int kMaxSplitBlocks = 64;  // blocks per model of a split launch: one lane each polls a block's slot
+constexpr int kMaxSplitIters = 1024;  // max_iter of a split launch: its exchange takes 8 bytes per block and iteration
 constexpr int kLatePolls = 1 << 13;  // split launch: polls before a workgroup looks for blocks that have none
 
 }  // namespace kyn

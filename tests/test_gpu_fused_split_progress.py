@@ -1,7 +1,7 @@
 """A split model's step ends, with the same bits, whatever share of its workgroups finds room on the
 GPU: launched with all of them, with one of each model (it then runs every block of the model) and
-with numbers between; with more blocks than the rotors' three; past the 64 blocks a split model
-may have (one workgroup then); and with two systems stepping at once from threads."""
+with numbers between; with more blocks than the rotors' three; past the 64 blocks and the 1024 iterations
+a split model may have (one workgroup then); and with two systems stepping at once from threads."""
 
 import ctypes as C
 import threading
@@ -93,6 +93,18 @@ def test_models_past_the_split_limit_keep_one_workgroup(kyn):
     # 21 copies of one rotor converge as one (the error is a mean over the degrees of freedom)
     one = q[1].get("q")
     assert np.max(np.abs(q[0].get("q").reshape(21, -1) - one.reshape(1, -1))) <= 1e-12 * np.max(np.abs(one))
+
+
+@pytest.mark.parametrize("max_iter,groups", [(1024, 3), (1025, 1), (1 << 24, 1)])
+def test_an_iteration_limit_past_the_exchange_is_taken_unsplit(kyn, max_iter, groups):
+    spec = _rotors([4])[0]
+    s = ota.KynSystem(kyn, spec, exec_mode=ota.EXEC_FUSED, max_iter=max_iter)
+    ref = ota.KynSystem(kyn, spec, exec_mode=ota.EXEC_FUSED)
+    assert (_launched(kyn, s), _launched(kyn, ref)) == (groups, 3)
+    for x in (s, ref):
+        assert x.step({}) == ota.KYN_OK
+    for a, b in zip(_state(s), _state(ref)):
+        assert np.array_equal(a, b)
 
 
 @PRECISIONS
