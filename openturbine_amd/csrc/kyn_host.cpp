@@ -252,6 +252,7 @@ struct kyn_system_s {
     std::vector<std::vector<int>> model_gdof_to_block_vec;  // per model: global dof -> rhs index
     std::vector<int> fused_work;  // the fused launch's list
     double* saved{};  // saved state (CopyStateData), on the device; allocated on first use
+    bool saved_on_host{false};  // in pinned host memory instead: the device had no room for it
     bool has_saved{false};
     // large blocks (library LU): block ids, sizes, matrix offsets, pivots, scratch vectors
     std::vector<int> large_blocks, large_n, large_nsys;
@@ -287,6 +288,7 @@ struct kyn_system_s {
         if (blas) (void)rocblas_destroy_handle(blas);
         if (stream) (void)hipStreamDestroy(stream);
         if (host_flags) (void)hipHostFree(host_flags);
+        if (saved_on_host) (void)hipHostFree(saved);
     }
 };
 
@@ -834,6 +836,16 @@ int guarded(F&& f) {
         return KYN_ERR_INVALID;
     }
 }
+
+// The system's device current for a scope (a caller may have another one current).
+struct OnDevice {
+    int before{0};
+    explicit OnDevice(int device) {
+        hip_check(hipGetDevice(&before), "hipGetDevice");
+        if (before != device) hip_check(hipSetDevice(device), "hipSetDevice");
+    }
+    ~OnDevice() { (void)hipSetDevice(before); }
+};
 
 double* field_ptr(kyn_system_s* s, int field, int& width) {
     auto& S = s->S;
@@ -2153,7 +2165,18 @@ int kyn_model_get_beam_element(kyn_model m, size_t elem, size_t* node_ids, doubl
 int kyn_save_state(kyn_system s) {
     return guarded([&] {
         if (!s) throw KynError(KYN_ERR_INVALID, "null system");
-        if (!s->saved) s->saved = s->arena.alloc<double>(kyn::state_copy_doubles(s->S));
+        const OnDevice on(s->device);
+        if (!s->saved) {
+            const size_t n = kyn::state_copy_doubles(s->S);
+            try {
+                s->saved = s->arena.alloc<double>(n);
+            } catch (const KynError&) {  // no room on the device: the copy kernel reaches pinned memory too
+                (void)hipGetLastError();
+                hip_check(hipHostMalloc(reinterpret_cast<void**>(&s->saved), n * sizeof(double), hipHostMallocDefault),
+                          "hipHostMalloc");
+                s->saved_on_host = true;
+            }
+        }
         kyn::launch_state_copy(s->S, s->saved, false, s->stream);
         hip_check(hipGetLastError(), "k_state_copy launch");
         hip_check(hipStreamSynchronize(s->stream), "sync");
@@ -2164,6 +2187,7 @@ int kyn_save_state(kyn_system s) {
 int kyn_restore_state(kyn_system s) {
     return guarded([&] {
         if (!s || !s->has_saved) throw KynError(KYN_ERR_INVALID, "no saved state");
+        const OnDevice on(s->device);
         kyn::launch_state_copy(s->S, s->saved, true, s->stream);
         hip_check(hipGetLastError(), "k_state_copy launch");
         hip_check(hipStreamSynchronize(s->stream), "sync");
