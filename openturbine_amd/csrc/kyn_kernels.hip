@@ -1010,8 +1010,9 @@ __device__ __forceinline__ void u_rows_group_fma(const float* Lc, float (&u)[kPa
 // 16 x 16 x 4 matrix-core products: A operand row lane % 16, k = lane / 16, B operand column
 // lane % 16, same k.  Both types accumulate c + a_0 b_0 + ... + a_3 b_3 like a chain of FMAs in
 // ascending k (the same bits on 5e6 random entries), so a trailing update on the matrix cores is
-// the update loop's FMA sequence; the mixed ensembles' states keep every bit (FP64 256 rotors, FP32
-// 1024, 6 steps).
+// the update loop's FMA sequence; the mixed FP64 ensemble's states keep every bit (256 rotors, 6
+// steps).  FP32 rotors factor without interchanges and do not come here; FP32 static solves and
+// blades on a hub node do, with residuals like LAPACK's FP32 LU of the same matrices.
 template <typename TT>
 struct MfmaTile;
 template <>
