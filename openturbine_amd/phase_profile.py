@@ -4,7 +4,10 @@ Loads the profiling build (libkynema_amd_phases.so: the same kernels with a time
 phase boundary of a block-iteration) and prints the mean shader cycles per block and Newton
 iteration for each phase.
 
-    python -m openturbine_amd.phase_profile --precision fp32 --rotors 512 --steps 2
+The default is large enough for the launch of one workgroup per model (small ensembles take one per
+block; the printed line says which).
+
+    python -m openturbine_amd.phase_profile --precision fp32 --rotors 1024 --steps 2
 """
 
 import argparse
@@ -26,7 +29,7 @@ def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--precision", choices=["fp32", "fp64"], default="fp32")
     ap.add_argument("--lib", default=str(LIB), help="profiling library to load (default: the in-tree build)")
-    ap.add_argument("--rotors", type=int, default=512)
+    ap.add_argument("--rotors", type=int, default=1024)
     ap.add_argument("--steps", type=int, default=2)
     ap.add_argument("--refine", type=int, default=0)
     ap.add_argument("--refine-bound", type=float, default=0.0,
@@ -51,8 +54,10 @@ def main():
     blocks_per_model = np.array([len(sp.beams) for sp in specs])
     count = int(((it1 - it0) * blocks_per_model).sum())
     total = 0.0
+    groups = C.c_int()
+    lib.L.kyn_debug_get_launch(s.h, C.byref(groups), None)
     print(f"{args.precision} refine {args.refine} (bound {args.refine_bound:g}), {args.rotors} rotors x {args.steps} steps, "
-          f"{count} block-iterations, step kernel {s.last_kernel_ms():.3f} ms")
+          f"{groups.value} workgroups, {count} block-iterations, step kernel {s.last_kernel_ms():.3f} ms")
     for i, name in enumerate(PHASES, start=1):
         c = ((a[i] - a[i - 1]) % (1 << 64)) / count
         total += c
@@ -61,7 +66,7 @@ def main():
     spans = ["LU wait for look-ahead (wave 0)", "LU wait + panel (wave 0)", "LU look-ahead + trailing (wave 1)",
              "LU panel steps incl. barrier", "refinement residual (HBM copy)", "refinement solve",
              "refinement forward sweep (wave 0)", "unpivoted LU: diagonal tile + L21", "unpivoted LU: U12 rows",
-             "unpivoted LU: MFMA trailing update","tU","tR"]
+             "unpivoted LU: MFMA trailing update"]
     for i, name in enumerate(spans):
         if i < 4 or a[16 + i]:
             print(f"    {name:34s} {a[16 + i] / count:10.0f} cycles")
