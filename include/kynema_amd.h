@@ -218,8 +218,9 @@ int kyn_debug_set_peer_wait_limit(kyn_system s, int polls);
  * No counterpart in the reference. */
 int kyn_debug_set_contraction_mask(kyn_system s, unsigned mask);
 /* Workgroups of the fused step's launch (one per model, or one per block where models are split) and
- * per element of the plain form's element kernel.  No counterpart in the reference. */
-int kyn_debug_get_launch(kyn_system s, int* fused_workgroups, int* element_workgroups);
+ * per element of the plain form's element kernel, and the CUs of the system's GPU; NULL skips.  No
+ * counterpart in the reference. */
+int kyn_debug_get_launch(kyn_system s, int* fused_workgroups, int* element_workgroups, int* compute_units);
 /* Launches the fused step with the workgroups of at most `per_model` blocks of every model (its last
  * ones): what a split step does when the others find no room on the GPU (tests).  No counterpart in
  * the reference. */

@@ -174,7 +174,7 @@ class KynLib:
         L.kyn_debug_set_wait_limit.argtypes = [C.c_void_p, C.c_int]
         L.kyn_debug_set_peer_wait_limit.argtypes = [C.c_void_p, C.c_int]
         L.kyn_debug_set_contraction_mask.argtypes = [C.c_void_p, C.c_uint]
-        L.kyn_debug_get_launch.argtypes = [C.c_void_p, C.POINTER(C.c_int), C.POINTER(C.c_int)]
+        L.kyn_debug_get_launch.argtypes = [C.c_void_p] + [C.POINTER(C.c_int)] * 3
         L.kyn_debug_set_fused_workgroups.argtypes = [C.c_void_p, C.c_int]
         L.kyn_get_element_terms.argtypes = [C.c_void_p, C.c_size_t, _dp, _dp]
         L.kyn_element_terms_noalloc.argtypes = [C.c_void_p, C.c_size_t, _dp, _dp]

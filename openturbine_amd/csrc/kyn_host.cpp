@@ -840,11 +840,16 @@ int guarded(F&& f) {
 // The system's device current for a scope (a caller may have another one current).
 struct OnDevice {
     int before{0};
+    bool changed{false};
     explicit OnDevice(int device) {
         hip_check(hipGetDevice(&before), "hipGetDevice");
-        if (before != device) hip_check(hipSetDevice(device), "hipSetDevice");
+        if (before == device) return;
+        hip_check(hipSetDevice(device), "hipSetDevice");
+        changed = true;
     }
-    ~OnDevice() { (void)hipSetDevice(before); }
+    ~OnDevice() {
+        if (changed) (void)hipSetDevice(before);
+    }
 };
 
 double* field_ptr(kyn_system_s* s, int field, int& width) {
@@ -2249,11 +2254,13 @@ int kyn_debug_set_peer_wait_limit(kyn_system s, int polls) {
     });
 }
 
-int kyn_debug_get_launch(kyn_system s, int* fused_workgroups, int* element_workgroups) {
+int kyn_debug_get_launch(kyn_system s, int* fused_workgroups, int* element_workgroups, int* compute_units) {
     return guarded([&] {
         if (!s) throw KynError(KYN_ERR_INVALID, "null system");
         if (fused_workgroups) *fused_workgroups = s->S.num_fused_work;
         if (element_workgroups) *element_workgroups = s->S.elem_split && s->S.precision == 0 ? 3 : 1;
+        if (compute_units)
+            hip_check(hipDeviceGetAttribute(compute_units, hipDeviceAttributeMultiprocessorCount, s->device), "attr");
         return KYN_OK;
     });
 }

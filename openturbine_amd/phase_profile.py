@@ -55,7 +55,7 @@ def main():
     count = int(((it1 - it0) * blocks_per_model).sum())
     total = 0.0
     groups = C.c_int()
-    lib.L.kyn_debug_get_launch(s.h, C.byref(groups), None)
+    lib.L.kyn_debug_get_launch(s.h, C.byref(groups), None, None)
     print(f"{args.precision} refine {args.refine} (bound {args.refine_bound:g}), {args.rotors} rotors x {args.steps} steps, "
           f"{groups.value} workgroups, {count} block-iterations, step kernel {s.last_kernel_ms():.3f} ms")
     for i, name in enumerate(PHASES, start=1):

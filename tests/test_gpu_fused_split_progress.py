@@ -47,8 +47,8 @@ def _system(kyn, specs, precision):
 
 
 def _launched(kyn, s):
-    fused, elem = C.c_int(), C.c_int()
-    assert kyn.L.kyn_debug_get_launch(s.h, C.byref(fused), C.byref(elem)) == ota.KYN_OK
+    fused = C.c_int()
+    assert kyn.L.kyn_debug_get_launch(s.h, C.byref(fused), None, None) == ota.KYN_OK
     return fused.value
 
 
