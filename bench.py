@@ -211,7 +211,7 @@ def structure_legs(lib, steps):
                      "failed_steps": fails}
         if name == "fp64":
             ms = kms / steps
-            out["element_kernel"] = {"kernel": "k_plain_element", "ms_per_launch": round(ms, 4),
+            out["element_kernel"] = {"kernel": "k_plain_element_split", "ms_per_launch": round(ms, 4),
                                      "algorithmic_bytes_per_launch": elem_bytes,
                                      "GB_s": round(elem_bytes / (ms / 1e3) / 1e9, 1)}
         log(f"  structure {name}: {steps} steps in {wall:.3f}s, {iters / steps:.1f} iters/step, fails {fails}")
