@@ -1012,7 +1012,8 @@ __device__ __forceinline__ void u_rows_group_fma(const float* Lc, float (&u)[kPa
 // ascending k (the same bits on 5e6 random entries), so a trailing update on the matrix cores is
 // the update loop's FMA sequence; the mixed FP64 ensemble's states keep every bit (256 rotors, 6
 // steps).  FP32 rotors factor without interchanges and do not come here; FP32 static solves and
-// blades on a hub node do, with residuals like LAPACK's FP32 LU of the same matrices.
+// blades on a hub node do: their increments keep the VALU form's bits too (18 to 143 dofs), with
+// residuals like those of LAPACK's FP32 LU of the same matrices.
 template <typename TT>
 struct MfmaTile;
 template <>
